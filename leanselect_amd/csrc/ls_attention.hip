@@ -7,8 +7,8 @@
 // j <= t + len_k - len_q when causal; all H/G heads of the group share the plan.
 //
 // Design (one workgroup per 24 query rows of one KV group and 16-head tile):
-//   * the plan row is turned into an ascending, duplicate-free page list with
-//     an LDS bitmap (ids past the causal frontier are dropped);
+//   * the plan rows are turned into an ascending, duplicate-free page list
+//     through an LDS table of row masks (ids past the causal frontier are dropped);
 //   * S^T = K . Q^T on v_mfma_f32_16x16x32: keys are MFMA rows, the 16 heads of
 //     the group are columns, so each lane owns one head and the online-softmax
 //     row statistics need only two cross-lane steps;
@@ -35,23 +35,6 @@
 #define LS_ATTN_MAX_PAGES 8192
 #define LS_ATTN_MAX_TAKE 128
 #define LS_ATTN_RING_TIMEOUT 1  // status bit: a ring wait expired (outputs invalid)
-
-__device__ __forceinline__ void ls_wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-__device__ __forceinline__ int ls_wave_excl_scan(int v, int lane, int* total) {
-  int x = v;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int y = __shfl_up(x, d, LS_WAVE);
-    if (lane >= d) x += y;
-  }
-  *total = __shfl(x, 63, LS_WAVE);
-  return x - v;
-}
 
 // pg_off[b] = sum_{b' < b} ceil(len_k(b') / 64): page-aligned start of each
 // sequence in the transposed V copy (in pages); tile_off[b] = sum_{b' < b}
@@ -106,7 +89,6 @@ __global__ void ls_attn_status_clear_kernel(int32_t* __restrict__ status) {
 #define LS_ATT_STAGES 4
 #define LS_ATT_KBYTES (64 * 256)             // K page: 64 rows x 256 B
 #define LS_ATT_STAGE_BYTES (2 * LS_ATT_KBYTES)  // + V^T page: 128 rows x 128 B
-#define LS_ATT_WORDS (LS_ATTN_MAX_PAGES / 32)
 #ifndef LS_ATT_XCD_CHUNK
 #define LS_ATT_XCD_CHUNK 16                  // consecutive tiles per XCD run
 #endif
@@ -116,7 +98,7 @@ __global__ void ls_attn_status_clear_kernel(int32_t* __restrict__ status) {
 #ifndef LS_ATT_SPIN_SLEEP
 #define LS_ATT_SPIN_SLEEP 1                  // s_sleep units between a waiting wave's polls
 #endif
-#define LS_ATT_UNION_CAP (64 * 64)           // union pages of a tile: one 64-bit need word per lane
+#define LS_ATT_UNION_CAP 4096                // union pages of a tile (ready tokens in the workspace)
 
 // Tile geometry for TPW rows per wave: rows per tile, the most ids per row it
 // accepts (so that its union fits LS_ATT_UNION_CAP) and the union bound.
@@ -127,7 +109,7 @@ struct LsAttTile {
       LS_ATTN_MAX_TAKE < LS_ATT_UNION_CAP / kTile ? LS_ATTN_MAX_TAKE : LS_ATT_UNION_CAP / kTile;
   static constexpr int kMaxUnion = kTile * kMaxTake;
   static_assert(kTile <= 32, "row masks are 32-bit");
-  static_assert(kMaxUnion <= LS_ATT_UNION_CAP, "one need word per lane");
+  static_assert(kMaxUnion <= LS_ATT_UNION_CAP, "one ready token per union page");
 };
 
 typedef _Float16 ls_half2 __attribute__((ext_vector_type(2)));
@@ -230,6 +212,16 @@ __device__ __forceinline__ float ls_sum_f16x2(uint32_t x, float acc) {
 }
 
 
+// What bounds it.  At two waves per SIMD the chunk math is a latency chain, not
+// an issue limit: a probe of the same instruction mix (16 MFMAs, 8 exponentials,
+// 24 other vector instructions) takes 150 ns per row-chunk with two waves, the
+// kernel took 245.  So the loop keeps a wave's waits off that chain: V^T is read
+// from LDS before the first row's Q K (and once for all rows), the second chunk's
+// K behind the first's softmax, the visit list and the ready word ahead of their
+// use, and the rare branches (causal frontier, rescale) out of line.  Attention
+// alone, same box, before -> after: 13.72 -> 12.19 ms (one 128K sequence, 64
+// pages), 4.00 -> 3.39 ms (32K, 96 pages, few shared), 1.55 -> 1.29 ms (four
+// sequences of 0.5K to 12K), 286 -> 234 us (4K), 3.99 -> 3.58 ms (32K with BIAS).
 // BIAS adds a per-key score bias (the NOSA eviction score, pre-scaled to base
 // 2): weight_j = 2^(scale_log2 * q.k_j + cb_j).  cb[g][64 pg_off[b] + j] is
 // staged like V^T and copied with each page (256 B per stage).
@@ -246,18 +238,18 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
   constexpr int D = 128;
   constexpr int TILE = LsAttTile<TPW>::kTile;
   constexpr int MAX_UNION = LsAttTile<TPW>::kMaxUnion;
-  constexpr int NEED_LANES = (MAX_UNION + 63) / 64;  // lanes holding a 64-bit need word
-  constexpr int NEED_WORDS = 2 * NEED_LANES;         // 32-bit need-mask words per wave
+  constexpr int MAX_VISITS = TPW * LsAttTile<TPW>::kMaxTake;  // pages of one wave
   constexpr uint32_t ROWS_MASK = (1u << TPW) - 1u;
-  // The per-row page bitmaps are only needed before streaming starts and
-  // share their LDS with the ring.
+  // The setup tables (rows per page, rows per union page) are only needed
+  // before streaming starts and share their LDS with the ring.
   __shared__ __align__(16) uint8_t s_ring[LS_ATT_STAGES * LS_ATT_STAGE_BYTES];
-  // Union entry: the mask of the tile rows that selected the page, and the page.
-  __shared__ uint32_t s_umeta[MAX_UNION];
+  uint32_t* s_rows = reinterpret_cast<uint32_t*>(s_ring);  // [page]: mask of the tile rows on it
+  uint32_t* s_umeta = s_rows + LS_ATTN_MAX_PAGES;          // [union page]: the same mask
   __shared__ uint16_t s_upage[MAX_UNION];
   __shared__ uint8_t s_uneed[MAX_UNION];  // waves with a row on the page
-  // Bit u of s_wneed[w] is set when a row of wave w selected union page u.
-  __shared__ uint32_t s_wneed[LS_ATT_WAVES][NEED_WORDS];
+  // The pages of each wave in the order it visits them: page | its rows on it
+  // << 13 | union index << 16.
+  __shared__ uint32_t s_wlist[LS_ATT_WAVES][MAX_VISITS];
   __shared__ int s_wsum[LS_ATT_WAVES];
   // Ring protocol: s_next = next union page to be claimed for copying;
   // s_rdy[st][0] = union index + 1 of the page whose copy into stage st has
@@ -266,15 +258,11 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
   __shared__ uint32_t s_next, s_done[LS_ATT_STAGES];
   __shared__ __align__(8) uint32_t s_rdy[LS_ATT_STAGES][2];
   __shared__ __align__(16) float s_bias[BIAS ? LS_ATT_STAGES * 64 : 4];
-  static_assert(TILE * LS_ATT_WORDS * 4 <= LS_ATT_STAGES * LS_ATT_STAGE_BYTES,
-                "page bitmaps must fit in the ring");
+  static_assert((LS_ATTN_MAX_PAGES + MAX_UNION) * 4 <= LS_ATT_STAGES * LS_ATT_STAGE_BYTES,
+                "the setup tables must fit in the ring");
   static_assert(TILE <= 32, "row masks are 32-bit");
-  static_assert(LS_ATT_WORDS <= LS_ATT_THREADS, "one bitmap word per thread");
-#ifdef LS_ATT_NO_ALIAS
-  __shared__ uint32_t s_bits[TILE][LS_ATT_WORDS];
-#else
-  uint32_t(*s_bits)[LS_ATT_WORDS] = reinterpret_cast<uint32_t(*)[LS_ATT_WORDS]>(s_ring);
-#endif
+  static_assert(LS_ATTN_MAX_PAGES <= 1 << 13 && TPW <= 3 && MAX_UNION <= 1 << 16,
+                "fields of a visit entry");
 
   const int tid = LS_TID;
   const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -313,14 +301,14 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
   const int64_t tile_jmax = row_jmax(n_rows - 1);
   const int last_page =
       tile_jmax >= 0 ? (int)min(tile_jmax / 64, (int64_t)LS_ATTN_MAX_PAGES - 1) : -1;
-  const int nwords = last_page / 32 + 1;
 
   // ---- per-row state: Q^T fragments (B operand), softmax stats, O^T ----
   // (the Q loads are issued first; they land while the page list is built)
   ls_u32x4 qf[TPW][4];
-  // m_run: running max in scaled base-2 units (score * scale_log2); thr: the
-  // raw score above which a key would exceed m_run by more than 2^8.
-  float m_run[TPW], l_run[TPW], thr[TPW];
+  // thr: the score (raw, or in base-2 units with a bias) above which a key would
+  // exceed the running maximum m = thr * scale_log2 - 8 (thr - 8 with a bias) by
+  // more than 2^8; m itself is not kept.
+  float l_run[TPW], thr[TPW];
   int jmax_r[TPW];
   ls_f32x4 o[TPW][8];
 #pragma unroll
@@ -333,7 +321,6 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
       qf[j][ks] = ls_load16(qrow + 32 * ks);
       if (!head_ok) qf[j][ks] = ls_u32x4{0u, 0u, 0u, 0u};
     }
-    m_run[j] = -INFINITY;
     l_run[j] = 0.f;
     thr[j] = -INFINITY;
     // Wave-uniform, so each chunk's row mask below is scalar work.
@@ -341,10 +328,11 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
 #pragma unroll
     for (int db = 0; db < 8; ++db) o[j][db] = ls_f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  // ---- per-row page bitmaps and their sorted union ----
-  for (int i = tid; i < TILE * nwords; i += LS_ATT_THREADS) s_bits[i / nwords][i % nwords] = 0u;
-  for (int i = tid; i < LS_ATT_WAVES * NEED_WORDS; i += LS_ATT_THREADS)
-    s_wneed[i / NEED_WORDS][i % NEED_WORDS] = 0u;
+  // ---- the tile's pages: rows per page, then their ascending union ----
+  // Every step works on 64 pages or ids per wave at a time: the tile's setup
+  // is exposed (one workgroup fills a CU's LDS), so it must not loop serially
+  // over a word's bits or a thread's pages.
+  for (int i = tid; i <= last_page; i += LS_ATT_THREADS) s_rows[i] = 0u;
   if (tid < LS_ATT_STAGES) {
     s_rdy[tid][0] = 0u;
     s_done[tid] = 0u;
@@ -353,32 +341,45 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
   __syncthreads();
   if (last_page >= 0) {
     const int32_t* ids = topk_idx + ((int64_t)g * total_q + t0) * take;
-    for (int i = tid; i < n_rows * take; i += LS_ATT_THREADS) {
-      const int row = i / take;
-      const int p = ids[i];
-      const int64_t jm = row_jmax(row);
-      if (p >= 0 && jm >= 0 && p <= jm / 64 && p <= last_page)
-        atomicOr(&s_bits[row][p >> 5], 1u << (p & 31));
+#pragma unroll
+    for (int j = 0; j < TPW; ++j) {
+      const int row = w * TPW + j;
+      const int pmax = jmax_r[j] >= 0 ? min(jmax_r[j] / 64, last_page) : -1;
+      if (row < n_rows)
+        for (int i = lane; i < take; i += 64) {
+          const int p = ids[(int64_t)row * take + i];
+          if (p >= 0 && p <= pmax) atomicOr(&s_rows[p], 1u << row);
+        }
     }
   }
   __syncthreads();
-  uint32_t word = 0u, row_word[TILE];
-#pragma unroll
-  for (int i = 0; i < TILE; ++i) {
-    row_word[i] = tid < nwords ? s_bits[i][tid] : 0u;
-    word |= row_word[i];
+  // Wave w counts, then places, the pages [w, w + 1) * seg64 of 64-page segments.
+  const int n_seg = (last_page + 64) / 64, seg_per = (n_seg + LS_ATT_WAVES - 1) / LS_ATT_WAVES;
+  const int seg0 = w * seg_per, seg1 = min(n_seg, seg0 + seg_per);
+  int wave_pages = 0;
+  for (int sg = seg0; sg < seg1; ++sg) {
+    const int p = 64 * sg + lane;
+    wave_pages += __popcll(__ballot(p <= last_page && s_rows[p] != 0u));
   }
-  int wtot;
-  const int wpos = ls_wave_excl_scan(__popc(word), lane, &wtot);
-  if (lane == 0) s_wsum[w] = wtot;
+  if (lane == 0) s_wsum[w] = wave_pages;
   __syncthreads();
-  int pos = wpos;
-  for (int i = 0; i < w; ++i) pos += s_wsum[i];
-  int n_union = 0;
+  int pos0 = 0, n_union = 0;
 #pragma unroll
-  for (int i = 0; i < LS_ATT_WAVES; ++i) n_union += s_wsum[i];
+  for (int i = 0; i < LS_ATT_WAVES; ++i) {
+    const int c = s_wsum[i];
+    pos0 += i < w ? c : 0;
+    n_union += c;
+  }
+  pos0 = __builtin_amdgcn_readfirstlane(pos0);
+  n_union = __builtin_amdgcn_readfirstlane(n_union);
   const int32_t* vexp_seq = vexp + (int64_t)g * n_pages_ws + pg_off[b];
-  const float inv_scale_log2 = 1.f / scale_log2;
+  // Wave-uniform floats are kept in scalar registers: with three rows of O and Q,
+  // the chunk's K and V^T fragments and a row's scores no vector register is spare.
+  auto uniform_f = [](float x) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(x)));
+  };
+  const float inv_scale_log2 = uniform_f(1.f / scale_log2);
+  auto run_max = [&](float t) { return BIAS ? t - 8.f : fmaf(t, scale_log2, -8.f); };
   // Page order.  Where the rows share many pages (at least
   // LS_ATT_SHARE_STRIDED / 10 plan ids per union page) the pages are visited in
   // a strided order (ascending page i goes to slot i * stride mod n_union, a
@@ -387,56 +388,45 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
   // waves over any window of pages.  Where they share few, ascending order:
   // the tiles running side by side on an XCD then reach a shared page at
   // nearly the same time, while it is still in that XCD's L2, and the waves'
-  // work is even anyway.  (Empty or one-page lists keep stride 1; a coprime
-  // odd stride below 64 + 7 exists for any list this kernel accepts, the loop
-  // bound only caps it.)
+  // work is even anyway.  The stride is the first odd number from 7 on that is
+  // coprime to n_union: 7, else 9, 11, 13 (15 shares the 3 that ruled 9 out),
+  // else 17 (a union that 3, 7, 11 and 13 divide is 3003 pages).
+  static_assert(MAX_UNION < 2 * 3003, "17 is coprime to a union that rules out the others");
   int stride = 1;
-  if (n_union > 1 && 10 * n_rows * take >= LS_ATT_SHARE_STRIDED * n_union) {
-    for (int cand = 7; cand < 71; cand += 2) {
-      int a = cand, b = n_union;
-      while (b) {
-        const int t = a % b;
-        a = b;
-        b = t;
-      }
-      if (a == 1) {
-        stride = cand;
-        break;
-      }
-    }
-  }
-  while (word) {
-    const int bit = __ffs(word) - 1;
-    word &= word - 1;
-    const int page = tid * 32 + bit;
-    uint32_t rows = 0u;
+  if (n_union > 1 && 10 * n_rows * take >= LS_ATT_SHARE_STRIDED * n_union)
+    stride = n_union % 7 ? 7 : n_union % 3 ? 9 : n_union % 11 ? 11 : n_union % 13 ? 13 : 17;
+  for (int sg = seg0; sg < seg1; ++sg) {
+    const int page = 64 * sg + lane;
+    const uint32_t rows = page <= last_page ? s_rows[page] : 0u;
+    const uint64_t mk = __ballot(rows != 0u);
+    const int pos = (int)__builtin_amdgcn_mbcnt_hi(
+        (uint32_t)(mk >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mk, (uint32_t)pos0));
+    if (rows != 0u) {
+      const int dst = (int)(((uint32_t)pos * (uint32_t)stride) % (uint32_t)n_union);
+      int n_waves = 0;
 #pragma unroll
-    for (int i = 0; i < TILE; ++i) rows |= ((row_word[i] >> bit) & 1u) << i;
-    const int dst = (int)(((uint32_t)pos * (uint32_t)stride) % (uint32_t)n_union);
-    int n_waves = 0;
-#pragma unroll
-    for (int i = 0; i < LS_ATT_WAVES; ++i) {
-      if (((rows >> (TPW * i)) & ROWS_MASK) != 0u) {
-        ++n_waves;
-        atomicOr(&s_wneed[i][dst >> 5], 1u << (dst & 31));
-      }
+      for (int i = 0; i < LS_ATT_WAVES; ++i) n_waves += ((rows >> (TPW * i)) & ROWS_MASK) != 0u;
+      s_umeta[dst] = rows;
+      s_upage[dst] = (uint16_t)page;
+      s_uneed[dst] = (uint8_t)n_waves;
     }
-    s_umeta[dst] = rows;
-    s_upage[dst] = (uint16_t)page;
-    s_uneed[dst] = (uint8_t)n_waves;
-    ++pos;
+    pos0 += __popcll(mk);
   }
-
-  __syncthreads();  // the union list is complete and the bitmaps are dead, so
-                    // the ring may be written
+  __syncthreads();
+  // This wave's pages, in union order.
+  int n_visits = 0;
+  for (int u0 = 0; u0 < n_union; u0 += 64) {
+    const int u = u0 + lane;
+    const uint32_t rows = u < n_union ? (s_umeta[u] >> (TPW * w)) & ROWS_MASK : 0u;
+    const uint64_t mk = __ballot(rows != 0u);
+    const int pos = (int)__builtin_amdgcn_mbcnt_hi(
+        (uint32_t)(mk >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mk, (uint32_t)n_visits));
+    if (rows != 0u) s_wlist[w][pos] = (uint32_t)s_upage[u] | rows << 13 | (uint32_t)u << 16;
+    n_visits += __popcll(mk);
+  }
+  __syncthreads();  // the lists are complete and the tables are dead, so the
+                    // ring may be written
   LS_WAIT_VMCNT(0);
-  // This wave's pages: bit b of lane l is set when one of its rows selected
-  // union page 64 l + b (the union holds at most 64 x 64 pages).
-  static_assert(NEED_LANES <= 64, "one need word per lane");
-  const uint64_t wneed =
-      lane < NEED_LANES
-          ? ((uint64_t)s_wneed[w][2 * lane + 1] << 32) | (uint64_t)s_wneed[w][2 * lane]
-          : 0ull;
 
   // ---- staging ----
   // One wave copies a whole union page into its stage: the page's staged
@@ -523,135 +513,125 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
     return (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)word) == (uint32_t)ui + 1u;
   };
 
-  auto compute_page = [&](int ui, int page, uint32_t sel, int v_e) {
-    const float p_unscale = __builtin_ldexpf(1.f, -v_e);
+  // K fragments of the chunk computed next.  The page's second chunk is read
+  // while the last row of the first still has its softmax and P V ahead of it:
+  // the fragments are dead once that row's Q K is issued, so this costs no
+  // register.  (Reading the next page's first chunk the same way, when it has
+  // already landed, measured 1-3% slower on every plan set.)
+  ls_u32x4 kf0[4], kf1[4];
+  auto load_k = [&](int ui, int c) {
     const uint8_t* kb = s_ring + (ui % LS_ATT_STAGES) * LS_ATT_STAGE_BYTES;
-    const uint8_t* vb = kb + LS_ATT_KBYTES;
+    const int R0 = 32 * c + r, R1 = 32 * c + 16 + r;
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const int base = 64 * page + 32 * c;
-      uint32_t need = 0;
-#pragma unroll
-      for (int j = 0; j < TPW; ++j) need |= (uint32_t)(((sel >> j) & 1u) && base <= jmax_r[j]) << j;
-      if (!need) continue;
-      // The chunk's K and V^T fragments are read once and shared by the rows.
-      const int R0 = 32 * c + r, R1 = 32 * c + 16 + r;
-      ls_u32x4 kf0[4], kf1[4], vf[8];
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        const int C = 4 * ks + q;
-        kf0[ks] = *reinterpret_cast<const ls_u32x4*>(kb + R0 * 256 + ((C ^ (R0 & 15)) << 4));
-        kf1[ks] = *reinterpret_cast<const ls_u32x4*>(kb + R1 * 256 + ((C ^ (R1 & 15)) << 4));
-      }
-      // V^T row 16 db + r (so (row >> 1) & 7 == (r >> 1) & 7), logical chunk 4c + q.
-      const uint8_t* vrow = vb + r * 128 + (((4 * c + q) ^ ((r >> 1) & 7)) << 4);
-      ls_f32x4 cbv0, cbv1;  // this lane's eight key biases (BIAS only)
-      if constexpr (BIAS) {
-        const float* bp = s_bias + (ui % LS_ATT_STAGES) * 64 + 32 * c + 8 * q;
-        cbv0 = *reinterpret_cast<const ls_f32x4*>(bp);
-        cbv1 = *reinterpret_cast<const ls_f32x4*>(bp + 4);
-      }
-      // S^T of one row: lane (r, q) gets head r's raw scores of keys base + 8q + 0..7.
-      auto qk = [&](int j, ls_f32x4& s0, ls_f32x4& s1) {
-        s0 = ls_f32x4{0.f, 0.f, 0.f, 0.f};
-        s1 = ls_f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-          s0 = LsElem<DT>::mfma(kf0[ks], qf[j][ks], s0);
-          s1 = LsElem<DT>::mfma(kf1[ks], qf[j][ks], s1);
-        }
-      };
-      // Online softmax update of row j with its chunk scores, then O^T += V^T P^T.
-      auto soft_pv = [&](int j, const ls_f32x4& s0, const ls_f32x4& s1) {
-        float sv[8] = {s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
-        if (base + 31 > jmax_r[j]) {  // the chunk crosses this row's causal frontier
-          // This lane's last visible key offset, formed here so that the eight
-          // key indices are not kept for every chunk (the empty asm keeps the
-          // compiler from rewriting the compares back into them).
-          int lim = jmax_r[j] - base - 8 * q;
-          asm("" : "+v"(lim));
-#pragma unroll
-          for (int i = 0; i < 8; ++i)
-            if (i > lim) sv[i] = -INFINITY;
-        }
-        // With a bias the scores are taken to base-2 units here (thr, m_run
-        // and the maxima below are then all in those units).
-        if constexpr (BIAS) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            sv[i] = fmaf(sv[i], scale_log2, cbv0[i]);
-            sv[4 + i] = fmaf(sv[4 + i], scale_log2, cbv1[i]);
-          }
-        }
-        // Plain maxima: the compiler inserts the wait states an MFMA result
-        // needs before a VALU read (it cannot for inline asm), and this file is
-        // built without IEEE NaN quieting, so they fuse into v_max3 (grouped
-        // here as three v_max3 and one v_max).
-        const float lmax = fmaxf(fmaxf(fmaxf(sv[6], sv[7]), fmaxf(fmaxf(sv[0], sv[1]), sv[2])),
-                                 fmaxf(fmaxf(sv[3], sv[4]), sv[5]));
-        // Rescale only when some head's max grows by more than 2^8 (or when the
-        // page's V scale leaves too little fp16 headroom for P up to 2^8).
-        if (__ballot(lmax > thr[j]) != 0ull || v_e > 7) {
-          float cm = lmax;
-          cm = fmaxf(cm, ls_shfl_xor(cm, 16));
-          cm = fmaxf(cm, ls_shfl_xor(cm, 32));
-          const float m_new = fmaxf(m_run[j], BIAS ? cm : cm * scale_log2);
-          const float alpha = __builtin_amdgcn_exp2f(m_run[j] - m_new);
-          m_run[j] = m_new;
-          thr[j] = BIAS ? m_new + 8.f : (m_new + 8.f) * inv_scale_log2;
-          l_run[j] *= alpha;
-#pragma unroll
-          for (int db = 0; db < 8; ++db) o[j][db] *= alpha;
-        }
-        // P' = P * 2^e (the page's V scale moved onto P, exact): one exp each;
-        // the row sum adds the fp16 P' that the MFMA uses, scaled back by 2^-e.
-        const float bias = (float)v_e - m_run[j];
-        ls_u32x4 pf;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if constexpr (BIAS)
-            pf[i] = ls_pack_f16x2(__builtin_amdgcn_exp2f(sv[2 * i] + bias),
-                                  __builtin_amdgcn_exp2f(sv[2 * i + 1] + bias));
-          else
-            pf[i] = ls_pack_f16x2(__builtin_amdgcn_exp2f(fmaf(sv[2 * i], scale_log2, bias)),
-                                  __builtin_amdgcn_exp2f(fmaf(sv[2 * i + 1], scale_log2, bias)));
-        }
-        const float lsum = ls_sum_f16x2(pf[3], ls_sum_f16x2(pf[2], ls_sum_f16x2(pf[1], ls_sum_f16x2(pf[0], 0.f))));
-        l_run[j] = fmaf(lsum, p_unscale, l_run[j]);
-        // The row's V^T fragments, read where they are used.
-#pragma unroll
-        for (int db = 0; db < 8; ++db) vf[db] = *reinterpret_cast<const ls_u32x4*>(vrow + db * 2048);
-#pragma unroll
-        for (int db = 0; db < 8; ++db) o[j][db] = LsElem<LS_F16>::mfma(vf[db], pf, o[j][db]);
-      };
-#pragma unroll
-      for (int j = 0; j < TPW; ++j) {
-        if (!((need >> j) & 1u)) continue;
-        ls_f32x4 s0, s1;
-        qk(j, s0, s1);
-        soft_pv(j, s0, s1);
-      }
+    for (int ks = 0; ks < 4; ++ks) {
+      const int C = 4 * ks + q;
+      kf0[ks] = *reinterpret_cast<const ls_u32x4*>(kb + R0 * 256 + ((C ^ (R0 & 15)) << 4));
+      kf1[ks] = *reinterpret_cast<const ls_u32x4*>(kb + R1 * 256 + ((C ^ (R1 & 15)) << 4));
     }
   };
 
-  // Next page of this wave: the lowest set need bit above `after` (n_union if none).
-  auto next_page = [&](int after) -> int {
-    const int from = after + 1, fl = from >> 6;
-    const uint64_t word = lane < fl ? 0ull : (lane == fl ? wneed & (~0ull << (from & 63)) : wneed);
-    const uint64_t lanes = __ballot(word != 0ull);
-    if (lanes == 0ull) return n_union;
-    const int L = (int)__builtin_ctzll(lanes);
-    const uint64_t wl = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(word >> 32), L) << 32) |
-                        (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)word, L);
-    return 64 * L + (int)__builtin_ctzll(wl);
+  // Chunk c (32 keys from key `base`) of the page in stage ui, for the rows in `need`.
+  auto chunk = [&](int ui, int c, int base, uint32_t need, int v_e, uint64_t ve_mask,
+                   float p_unscale) {
+    // V^T row 16 db + r (so (row >> 1) & 7 == (r >> 1) & 7), logical chunk 4c + q;
+    // read once for all rows, in flight during the first row's Q K and softmax.
+    const uint8_t* vrow = s_ring + (ui % LS_ATT_STAGES) * LS_ATT_STAGE_BYTES + LS_ATT_KBYTES +
+                          r * 128 + (((4 * c + q) ^ ((r >> 1) & 7)) << 4);
+    ls_u32x4 vf[8];
+#pragma unroll
+    for (int db = 0; db < 8; ++db) vf[db] = *reinterpret_cast<const ls_u32x4*>(vrow + db * 2048);
+#pragma unroll
+    for (int j = 0; j < TPW; ++j) {
+      if (!((need >> j) & 1u)) continue;
+      // S^T: lane (r, q) gets head r's raw scores of keys base + 8q + 0..7.
+      ls_f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        s0 = LsElem<DT>::mfma(kf0[ks], qf[j][ks], s0);
+        s1 = LsElem<DT>::mfma(kf1[ks], qf[j][ks], s1);
+      }
+      if (c == 0 && (need >> (j + 1)) == 0u) load_k(ui, 1);
+      float sv[8] = {s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
+      if (__builtin_expect(base + 31 > jmax_r[j], 0)) {  // the chunk crosses this row's causal frontier
+        // This lane's last visible key offset, formed here so that the eight
+        // key indices are not kept for every chunk (the empty asm keeps the
+        // compiler from rewriting the compares back into them).
+        int lim = jmax_r[j] - base - 8 * q;
+        asm("" : "+v"(lim));
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (i > lim) sv[i] = -INFINITY;
+      }
+      // With a bias the scores are taken to base-2 units here (thr and the
+      // maxima below are then all in those units).
+      if constexpr (BIAS) {
+        const float* bp = s_bias + (ui % LS_ATT_STAGES) * 64 + 32 * c + 8 * q;
+        const ls_f32x4 cbv0 = *reinterpret_cast<const ls_f32x4*>(bp);
+        const ls_f32x4 cbv1 = *reinterpret_cast<const ls_f32x4*>(bp + 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          sv[i] = fmaf(sv[i], scale_log2, cbv0[i]);
+          sv[4 + i] = fmaf(sv[4 + i], scale_log2, cbv1[i]);
+        }
+      }
+      // Plain maxima: the compiler inserts the wait states an MFMA result
+      // needs before a VALU read (it cannot for inline asm), and this file is
+      // built without IEEE NaN quieting, so they fuse into v_max3 (grouped
+      // here as three v_max3 and one v_max).
+      const float lmax = fmaxf(fmaxf(fmaxf(sv[6], sv[7]), fmaxf(fmaxf(sv[0], sv[1]), sv[2])),
+                               fmaxf(fmaxf(sv[3], sv[4]), sv[5]));
+      // Rescale only when some head's max grows by more than 2^8 (or when the
+      // page's V scale leaves too little fp16 headroom for P up to 2^8).
+      if (__builtin_expect((__ballot(lmax > thr[j]) | ve_mask) != 0ull, 0)) {
+        float cm = lmax;
+        cm = fmaxf(cm, ls_shfl_xor(cm, 16));
+        cm = fmaxf(cm, ls_shfl_xor(cm, 32));
+        const float m_old = run_max(thr[j]);
+        const float m_new = fmaxf(m_old, BIAS ? cm : cm * scale_log2);
+        thr[j] = BIAS ? m_new + 8.f : (m_new + 8.f) * inv_scale_log2;
+        const float alpha = __builtin_amdgcn_exp2f(m_old - run_max(thr[j]));
+        l_run[j] *= alpha;
+#pragma unroll
+        for (int db = 0; db < 8; ++db) o[j][db] *= alpha;
+      }
+      // P' = P * 2^e (the page's V scale moved onto P, exact): one exp each;
+      // the row sum adds the fp16 P' that the MFMA uses, scaled back by 2^-e.
+      const float bias = BIAS ? (float)(v_e + 8) - thr[j]
+                              : fmaf(-scale_log2, thr[j], (float)(v_e + 8));
+      ls_u32x4 pf;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if constexpr (BIAS)
+          pf[i] = ls_pack_f16x2(__builtin_amdgcn_exp2f(sv[2 * i] + bias),
+                                __builtin_amdgcn_exp2f(sv[2 * i + 1] + bias));
+        else
+          pf[i] = ls_pack_f16x2(__builtin_amdgcn_exp2f(fmaf(sv[2 * i], scale_log2, bias)),
+                                __builtin_amdgcn_exp2f(fmaf(sv[2 * i + 1], scale_log2, bias)));
+      }
+      const float lsum = ls_sum_f16x2(pf[3], ls_sum_f16x2(pf[2], ls_sum_f16x2(pf[1], ls_sum_f16x2(pf[0], 0.f))));
+      l_run[j] = fmaf(lsum, p_unscale, l_run[j]);
+#pragma unroll
+      for (int db = 0; db < 8; ++db) o[j][db] = LsElem<LS_F16>::mfma(vf[db], pf, o[j][db]);
+    }
   };
-  // The next page's union entry is read before the current page is computed.
-  int ui = next_page(-1);
-  uint32_t meta = ui < n_union ? s_umeta[ui] : 0u;
-  int page_cur = ui < n_union ? (int)s_upage[ui] : 0;
+
+  // A visit's list entry is read two visits ahead and its stage word during
+  // the visit before, so that neither read is waited for where the page is ready: a page
+  // stays in its stage until this wave is done with it, so a word that showed
+  // its token once stays valid, and LDS accesses of a wave are in order, so the
+  // page's data is read after it.
+  auto entry = [&](int k) -> uint32_t { return k < n_visits ? s_wlist[w][k] : 0u; };
+  auto uniform = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); };
+  auto stage_peek = [&](int ui) -> uint64_t {
+    return __hip_atomic_load(reinterpret_cast<uint64_t*>(&s_rdy[ui % LS_ATT_STAGES][0]),
+                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  };
+  uint32_t e_cur = uniform(entry(0));
+  uint32_t e_next = entry(1);
+  uint64_t sw = stage_peek((int)(e_cur >> 16));
   int spins = spin_limit;  // bound of this wave's next wait (in polls)
-  while (ui < n_union) {
-    uint64_t sw = stage_word(ui);
+  for (int k = 0; k < n_visits; ++k) {
+    const int ui = (int)(e_cur >> 16);
     if (!is_ready(ui, sw)) {
       // Bounded wait (the protocol cannot deadlock; the bound only guarantees
       // that a wave always finishes).  A wave whose wait expires reports it
@@ -675,20 +655,28 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
                                 __HIP_MEMORY_SCOPE_AGENT);
       }
     }
-
-    const int nxt = next_page(ui);
-    const uint32_t meta_next = nxt < n_union ? s_umeta[nxt] : 0u;
-    const int page_next = nxt < n_union ? (int)s_upage[nxt] : 0;
-    const uint32_t m = (uint32_t)__builtin_amdgcn_readfirstlane((int)meta);
-    compute_page(ui, __builtin_amdgcn_readfirstlane(page_cur), (m >> (TPW * w)) & ROWS_MASK,
-                 __builtin_amdgcn_readfirstlane((int)(uint32_t)(sw >> 32)));
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int v_e = __builtin_amdgcn_readfirstlane((int)(uint32_t)(sw >> 32));
+    const uint32_t e = e_cur;
+    e_cur = uniform(e_next);
+    e_next = entry(k + 2);
+    const int page = (int)(e & 0x1fffu);
+    const uint32_t sel = (e >> 13) & ROWS_MASK;
+    const float p_unscale = uniform_f(__builtin_ldexpf(1.f, -v_e));
+    const uint64_t ve_mask = v_e > 7 ? ~0ull : 0ull;
+    load_k(ui, 0);
+    // Every row of the entry sees the page's first chunk.
+    chunk(ui, 0, 64 * page, sel, v_e, ve_mask, p_unscale);
+    uint32_t need = 0;
+#pragma unroll
+    for (int j = 0; j < TPW; ++j)
+      need |= (uint32_t)(((sel >> j) & 1u) && 64 * page + 32 <= jmax_r[j]) << j;
+    sw = stage_peek((int)(e_cur >> 16));
+    if (need) chunk(ui, 1, 64 * page + 32, need, v_e, ve_mask, p_unscale);
     // Done with the stage (the release orders this wave's reads of it first).
     if (lane == 0)
       __hip_atomic_fetch_add(&s_done[ui % LS_ATT_STAGES], 1u, __ATOMIC_RELEASE,
                              __HIP_MEMORY_SCOPE_WORKGROUP);
-    ui = nxt;
-    meta = meta_next;
-    page_cur = page_next;
   }
   LS_WAIT_VMCNT(0);  // no copy of this wave may land after the workgroup ends
 
@@ -723,7 +711,7 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
     }
     if (lse && q == 0)
       lse[((int64_t)g * gs + head) * total_q + t] =
-          l_tot > 0.f ? m_run[j] * 0.69314718055994531f + __logf(l_tot) : INFINITY;
+          l_tot > 0.f ? run_max(thr[j]) * 0.69314718055994531f + __logf(l_tot) : INFINITY;
   }
 }
 
