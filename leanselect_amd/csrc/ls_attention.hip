@@ -23,6 +23,7 @@
 #include "ls_common.h"
 
 #include <mutex>
+#include <type_traits>
 
 // Work-item and workgroup ids straight from the hardware: this file is built
 // without IEEE NaN quieting, and the device library's id helpers (built with
@@ -72,8 +73,7 @@ __global__ void ls_attn_status_clear_kernel(int32_t* __restrict__ status) {
 // ---------------------------------------------------------------------------
 // Tile kernel: one workgroup = 8 x TPW consecutive query rows of one sequence
 // and one KV group for 16 of its query heads (8 waves x TPW rows, two waves per
-// SIMD; the launcher uses TPW = 3, 24-row tiles, for every plan of up to
-// LS_ATTN_MAX_TAKE ids).  The rows' page plans are OR-ed into a union page list;
+// SIMD; the launcher picks TPW).  The rows' page plans are OR-ed into a union page list;
 // each union page of staged K and V^T is streamed once into a 4-stage LDS ring
 // with direct global->LDS loads, and every row that selected the page runs its
 // MFMAs on it.  Rows that did not select a page skip it (no masked-out work).
@@ -89,9 +89,6 @@ __global__ void ls_attn_status_clear_kernel(int32_t* __restrict__ status) {
 #define LS_ATT_STAGES 4
 #define LS_ATT_KBYTES (64 * 256)             // K page: 64 rows x 256 B
 #define LS_ATT_STAGE_BYTES (2 * LS_ATT_KBYTES)  // + V^T page: 128 rows x 128 B
-#ifndef LS_ATT_XCD_CHUNK
-#define LS_ATT_XCD_CHUNK 16                  // consecutive tiles per XCD run
-#endif
 #ifndef LS_ATT_SHARE_STRIDED
 #define LS_ATT_SHARE_STRIDED 25              // plan ids per union page (x10) for the strided order
 #endif
@@ -234,7 +231,7 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
     const int32_t* __restrict__ pg_off, const int32_t* __restrict__ tile_off, int batch,
     int64_t total_q, int G, int gs, const int32_t* __restrict__ topk_idx, int take,
     float scale_log2, int causal, uint16_t* __restrict__ out, float* __restrict__ lse,
-    int per_xcd, int32_t* __restrict__ status, int spin_limit) {
+    int run, int span, int per_xcd, int32_t* __restrict__ status, int spin_limit) {
   constexpr int D = 128;
   constexpr int TILE = LsAttTile<TPW>::kTile;
   constexpr int MAX_UNION = LsAttTile<TPW>::kMaxUnion;
@@ -269,19 +266,20 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
   const int r = lane & 15, q = lane >> 4;
 
   // XCD-aware tile order.  Consecutive workgroups land on different XCDs
-  // (workgroup x runs on XCD x % 8).  Each XCD takes runs of LS_ATT_XCD_CHUNK
-  // consecutive tiles, so the tiles in flight on one XCD are neighbours that
-  // share pages in its L2, and the runs go round-robin over the XCDs, so every
-  // XCD gets an even share of early (small-union) and late (large-union) rows.
-  // Runs are taken from the end of the sequence first: the largest tiles
-  // start first and small ones fill the tail.  The grid is a multiple of
-  // 8 * LS_ATT_XCD_CHUNK, so this is a permutation of the workgroup indices.
-  const int64_t xi = LS_BID_X / 8;
+  // (workgroup x runs on XCD x % 8).  Each XCD takes runs of `run` consecutive
+  // tiles, so the tiles in flight on one XCD are neighbours that share pages in
+  // its L2, and turns to the next KV group every `span` tiles (a multiple of
+  // run).  The runs are dealt over the XCDs there and back (0..7, then 7..0), and
+  // from the end of the sequence first, so every XCD gets an even share of late
+  // (large-union) and early (small-union) rows, the largest tiles start first and
+  // small ones fill the tail.  The grid is 8 * G * (a multiple of span), so this
+  // is a permutation of the workgroup indices.
+  const int xcd = LS_BID_X % 8, xi = LS_BID_X / 8;
+  const int turn = xi / span, g = turn % G, at = turn / G * span + xi % span;
+  const int deal = at / run;
   const int64_t tile = 8LL * per_xcd - 1 -
-                       ((xi / LS_ATT_XCD_CHUNK) * (8 * LS_ATT_XCD_CHUNK) +
-                        (int64_t)(LS_BID_X % 8) * LS_ATT_XCD_CHUNK + xi % LS_ATT_XCD_CHUNK);
+                       ((int64_t)(8 * deal + ((deal & 1) ? 7 - xcd : xcd)) * run + at % run);
   if (tile >= tile_off[batch]) return;
-  const int g = LS_BID_Y;
   const int head = LS_BID_Z * 16 + r;
   const bool head_ok = head < gs;
 
@@ -762,6 +760,39 @@ AttnWs attn_ws(int64_t total_k, int batch, int G, bool bias) {
   return L;
 }
 
+// How a call's rows are cut into tiles and dealt to the XCDs: rows per wave of a
+// tile, consecutive tiles per XCD run, tiles of one KV group an XCD takes before
+// it turns to the next group, and tiles of one group per XCD.
+struct AttnTiling {
+  int tpw, run, span, per_xcd;
+};
+
+// One workgroup fills a CU's LDS, so a call runs in rounds of 256 tiles.  Three
+// rows a wave (24-row tiles) share each page copy among the most rows, but a call
+// of few rows then leaves CUs idle, or a second round nearly empty: while the
+// smaller tile still gives at most two rounds it is the faster one (attention of
+// one sequence, us, tiles of 8 / 16 / 24 rows: 600 rows 28 / 36 / 44, 2000 70 / 79
+// / 98, 2300 91 / 88 / 107, 4096 194 / 156 / 178, 4700 255 / 210 / 200).  Runs of 4
+// tiles even the XCDs' loads where runs of 16 leave some idle (8K rows 411 against
+// 463 us, 4096 rows 174 against 210) and cost nothing at 128K (12.06 against
+// 12.08 ms).  An XCD that alternates between the KV groups run by run starts every
+// group's large tiles early, which a call of up to four rounds needs (three
+// sequences of 4500 rows 106 against 134 us); longer calls keep to one group at a
+// time, whose pages then have the XCD's L2 to themselves (128K 12.06 against 12.42
+// ms, four sequences of 24K rows 1.20 against 1.25).
+AttnTiling attn_tiling(int64_t total_q, int batch, int G, int head_tiles) {
+  constexpr int64_t kCus = 256;
+  auto tiles = [&](int tpw) { return (total_q + LS_ATT_WAVES * tpw - 1) / (LS_ATT_WAVES * tpw); };
+  const int64_t per_tile = (int64_t)G * head_tiles;
+  AttnTiling t;
+  t.tpw = tiles(1) * per_tile <= 2 * kCus ? 1 : tiles(2) * per_tile <= 2 * kCus ? 2 : 3;
+  t.run = 4;
+  const int64_t bound = tiles(t.tpw) + batch;  // each sequence's last tile may be partial
+  t.per_xcd = (int)(t.run * ((bound + 8 * t.run - 1) / (8 * t.run)));
+  t.span = tiles(t.tpw) * per_tile <= 4 * kCus ? t.run : t.per_xcd;
+  return t;
+}
+
 template <int DT, bool BIAS, int TPW>
 void launch_tile(dim3 grid, hipStream_t s, const void* q, int64_t q_rs, const uint8_t* kv,
                  const AttnWs& L, const int32_t* vexp, const float* cb,
@@ -769,11 +800,11 @@ void launch_tile(dim3 grid, hipStream_t s, const void* q, int64_t q_rs, const ui
                  const int32_t* cu_q, const int32_t* cu_k, const int32_t* pg,
                  const int32_t* tiles, int batch, int64_t total_q, int G, int gs,
                  const int32_t* topk_idx, int take, float scale_log2, int causal, void* out,
-                 float* lse, int32_t* status) {
+                 float* lse, const AttnTiling& tl, int32_t* status) {
   hipLaunchKernelGGL((ls_attn_tile_kernel<DT, BIAS, TPW>), grid, dim3(LS_ATT_THREADS), 0, s,
                      (const uint16_t*)q, q_rs, kv, L.lpad, vexp, cb, tok,
                      L.n_pages, cu_q, cu_k, pg, tiles, batch, total_q, G, gs, topk_idx, take,
-                     scale_log2, causal, (uint16_t*)out, lse, (int)(grid.x / 8), status,
+                     scale_log2, causal, (uint16_t*)out, lse, tl.run, tl.span, tl.per_xcd, status,
                      g_spin_limit);
 }
 
@@ -822,10 +853,9 @@ int attn_run(const char* who, const void* q, int64_t q_row_stride, const void* k
   float* cb = bias ? (float*)(ws + L.cb) : nullptr;
   int32_t* tok = (int32_t*)(ws + L.tok);
   int32_t* status = status_out ? status_out : (int32_t*)(ws + L.status);
-  // 24-row tiles (three rows a wave): their union bound holds every plan accepted.
-  constexpr int kTpw = 3;
-  static_assert(LsAttTile<kTpw>::kMaxTake >= LS_ATTN_MAX_TAKE, "every accepted plan fits a tile");
-  const int tile_rows = LsAttTile<kTpw>::kTile;
+  const int gs = num_heads / num_kv_heads;
+  const AttnTiling tl = attn_tiling(total_q, batch, num_kv_heads, (gs + 15) / 16);
+  const int tile_rows = LS_ATT_WAVES * tl.tpw;
   hipLaunchKernelGGL(ls_attn_plan_kernel, dim3(1), dim3(64), 0, s, cu_seqlens_q, cu_seqlens_k,
                      batch, tile_rows, pg, tiles, tok, LS_ATT_UNION_CAP + 1, status);
   int rc = ls_check_launch("ls_attn_plan_kernel");
@@ -854,24 +884,27 @@ int attn_run(const char* who, const void* q, int64_t q_row_stride, const void* k
       if ((rc = ls_check_launch("ls_bias_kernel"))) return rc;
     }
   }
-  const int gs = num_heads / num_kv_heads;
   const float scale = softmax_scale > 0.f ? softmax_scale : 1.0f / sqrtf((float)head_dim);
   const float scale_log2 = scale * 1.4426950408889634f;
-  const int64_t tile_bound = (total_q + tile_rows - 1) / tile_rows + batch;
-  constexpr int64_t kRound = 8 * LS_ATT_XCD_CHUNK;  // whole runs on every XCD
-  const dim3 grid((unsigned)(kRound * ((tile_bound + kRound - 1) / kRound)), num_kv_heads,
-                  (gs + 15) / 16);
+  const dim3 grid((unsigned)(8 * tl.per_xcd * num_kv_heads), 1, (gs + 15) / 16);
 #define LS_TILE_ARGS                                                                              \
   grid, s, q, q_row_stride, kv, L, vexp, cb, tok, cu_seqlens_q, cu_seqlens_k, pg,              \
       tiles, batch, total_q, num_kv_heads, gs, topk_idx, take, scale_log2, causal, out, lse, \
-      status
-  if (dtype == LS_BF16) {
-    if (bias) launch_tile<LS_BF16, true, kTpw>(LS_TILE_ARGS);
-    else launch_tile<LS_BF16, false, kTpw>(LS_TILE_ARGS);
-  } else {
-    if (bias) launch_tile<LS_F16, true, kTpw>(LS_TILE_ARGS);
-    else launch_tile<LS_F16, false, kTpw>(LS_TILE_ARGS);
-  }
+      tl, status
+  auto launch = [&](auto tpw) {
+    constexpr int kTpw = decltype(tpw)::value;
+    static_assert(LsAttTile<kTpw>::kMaxTake >= LS_ATTN_MAX_TAKE, "every accepted plan fits a tile");
+    if (dtype == LS_BF16) {
+      if (bias) launch_tile<LS_BF16, true, kTpw>(LS_TILE_ARGS);
+      else launch_tile<LS_BF16, false, kTpw>(LS_TILE_ARGS);
+    } else {
+      if (bias) launch_tile<LS_F16, true, kTpw>(LS_TILE_ARGS);
+      else launch_tile<LS_F16, false, kTpw>(LS_TILE_ARGS);
+    }
+  };
+  if (tl.tpw == 1) launch(std::integral_constant<int, 1>());
+  else if (tl.tpw == 2) launch(std::integral_constant<int, 2>());
+  else launch(std::integral_constant<int, 3>());
 #undef LS_TILE_ARGS
   return ls_check_launch("ls_attn_tile_kernel");
 }

@@ -237,6 +237,34 @@ def test_attention_every_row_of_a_ragged_batch():
     _check_attention(case, ids, list(range(case.cu_host[-1])))
 
 
+@pytest.mark.parametrize("lens", [(1,), (9, 1, 40), (2048,), (2049,), (4095, 1), (4097,),
+                                  (12288,), (12289,), (2000, 1000, 1500)])
+@pytest.mark.parametrize("biased", [False, True])
+def test_attention_tile_sizes_and_tile_deal(lens, biased):
+    """Calls on both sides of the launcher's lines between 8-, 16- and 24-row tiles
+    (two KV groups: 2048 and 4096 rows) and between the two orders of the tile deal
+    (12288 rows): every row is written, and sampled rows match the oracle, with and
+    without the NOSA key bias."""
+    case, ids = _attention_case(lens=lens, seed=14)
+    rows = spread_rows(case.cu_host, per_seq=24)
+    out = torch.full_like(case.q, float("nan"))
+    if biased:
+        gen = torch.Generator(device=DEV).manual_seed(15)
+        cis = torch.randn(case.cu_host[-1], 2, generator=gen, device=DEV).to(case.q.dtype)
+        out = nosa_sparse_attention(case.q, case.k, case.v, cis, case.cu_seqlens, case.cu_seqlens,
+                                    case.max_seqlen, case.max_seqlen, ids)
+        want = oracle.nosa_attention(case.q.cpu(), case.k.cpu(), case.v.cpu(), cis.cpu(),
+                                     case.cu_host, case.cu_host, ids.cpu()[:, rows], rows=rows,
+                                     ids_rows_aligned=True)
+        ok, mx, mr = oracle.check_attention(out.cpu()[rows], want)
+        assert ok, (mx, mr)
+    else:
+        sparse_attention(case.q, case.k, case.v, case.cu_seqlens, case.cu_seqlens,
+                         case.max_seqlen, case.max_seqlen, ids, out=out)
+        _check_attention(case, ids, rows)
+    assert bool(torch.isfinite(out).all())
+
+
 def test_attention_messy_ids_duplicates_unsorted_out_of_range():
     case, ids = _attention_case(lens=(1500,), seed=7)
     g = torch.Generator(device="cpu").manual_seed(0)
