@@ -597,6 +597,23 @@ int ls_sparse_attn_kvcache(const void* q, int64_t q_row_stride, const int32_t* c
                            int32_t causal, int32_t n_splits, void* out, float* softmax_lse,
                            void* workspace, size_t workspace_bytes, void* stream);
 
+/*
+ * The same over every cached page (no plan, any number of pages): row i of
+ * sequence b attends all keys j < cache_seqlens[b] (causal = 0) or j <=
+ * cache_seqlens[b] - len_q(b) + i (causal = 1); each row's visible pages are
+ * cut evenly over its n_splits slices.  Workspace from
+ * ls_sparse_attn_kvcache_workspace_size.
+ * Replaces infllmv2_attn_with_kvcache without topk_idx
+ * (third_party/infllmv2/paper1.patch:2511-2615).
+ */
+int ls_dense_attn_kvcache(const void* q, int64_t q_row_stride, const int32_t* cu_seqlens_q,
+                          int64_t total_q, const void* k_cache, const void* v_cache,
+                          int64_t cache_batch_stride, int64_t cache_row_stride,
+                          const int32_t* cache_seqlens, int32_t batch, int32_t num_heads,
+                          int32_t num_kv_heads, int32_t head_dim, int32_t dtype,
+                          float softmax_scale, int32_t causal, int32_t n_splits, void* out,
+                          float* softmax_lse, void* ws, size_t ws_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -106,6 +106,9 @@ SIGNATURES = {
     "ls_sparse_attn_kvcache": (
         _i32, [_p, _i64, _p, _i64, _p, _p, _i64, _i64, _p, _i32, _i32, _i32, _i32, _i32, _p,
                _i32, _f32, _i32, _i32, _p, _p, _p, _sz, _p]),
+    "ls_dense_attn_kvcache": (
+        _i32, [_p, _i64, _p, _i64, _p, _p, _i64, _i64, _p, _i32, _i32, _i32, _i32, _i32, _f32,
+               _i32, _i32, _p, _p, _p, _sz, _p]),
 }
 
 _lib = None

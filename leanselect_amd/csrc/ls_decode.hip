@@ -603,7 +603,8 @@ __global__ __launch_bounds__(256) void ls_decode_topk_wg_kernel(
 // a 16-bit head and a 16-bit remainder (two MFMAs) so it carries about 16
 // significant bits; V^T fragments come from the wave's LDS copy of the page.
 // ---------------------------------------------------------------------------
-#define LS_DEC_VPITCH 260  // bytes per staged V row (65 dwords: conflict-free transposed reads)
+#define LS_DEC_VPITCH 264  // bytes per staged V row: 8-byte stores; 8 rows are 16 banks apart, so the
+                           // transposed reads of the four lane groups hit distinct banks
 #define LS_DEC_VBYTES (64 * LS_DEC_VPITCH)
 #define LS_DEC_PART (16 * 128 + 32)  // floats per partial: O [16][128], m [16], l [16]
 #define LS_DEC_MAX_SPLITS 64
@@ -615,7 +616,17 @@ __device__ __forceinline__ void ls_dec_wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <int DT>
+//
+// A wave's pages are pipelined: the next page's K rows are loaded as soon as this
+// page's Q K has read them, its V rows as soon as this page's are in LDS, so a
+// wave's second page does not wait for memory again (no register is added: the
+// loads reuse the fragments they follow).
+// Bound by memory latency at one or two pages a wave, then by the waves' serial
+// page time.  Attention and combine, before -> after: 26.0 -> 21.6 us at four
+// pages a wave (one row of 64 pages, 4 splits), 22.0 -> 21.2 us at two (16 rows).
+// DENSE: every page of the row's cache instead of a plan (topk_idx unused); the
+// row's own visible pages are cut evenly over the waves of its splits.
+template <int DT, bool DENSE>
 __global__ __launch_bounds__(256) void ls_decode_attn_kernel(
     const uint16_t* __restrict__ q, int64_t qrs, const int32_t* __restrict__ cu_q, int batch,
     int64_t total_q, const uint16_t* __restrict__ kc_, const uint16_t* __restrict__ vc_,
@@ -625,7 +636,8 @@ __global__ __launch_bounds__(256) void ls_decode_attn_kernel(
   const int s = LS_BID_X;
   const int64_t t = LS_BID_Y;
   const int g = LS_BID_Z;
-  const int tid = LS_TID, lane = tid & 63, w = tid >> 6;
+  const int tid = LS_TID, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, qg = lane >> 4;
   __shared__ __attribute__((aligned(16))) uint8_t s_v[4][LS_DEC_VBYTES];
   uint8_t* sv_w = s_v[w];
@@ -645,44 +657,82 @@ __global__ __launch_bounds__(256) void ls_decode_attn_kernel(
   ls_f32x4 o[8];
 #pragma unroll
   for (int db = 0; db < 8; ++db) o[db] = ls_f32x4{0.f, 0.f, 0.f, 0.f};
-  // The row's plan ids, 64 per register (topk <= 64 * LS_DEC_ID_REGS).
-  const int32_t* idrow = topk_idx + ((int64_t)g * total_q + t) * topk;
-  int idr[LS_DEC_ID_REGS];
-#pragma unroll
-  for (int k = 0; k < LS_DEC_ID_REGS; ++k) idr[k] = 64 * k + lane < topk ? idrow[64 * k + lane] : -1;
   const uint16_t* kseq = kc_ + (int64_t)b * cbs + (int64_t)g * D;
   const uint16_t* vseq = vc_ + (int64_t)b * cbs + (int64_t)g * D;
-  const int slot0 = (4 * s + w) * ppw, slot1 = min(topk, slot0 + ppw);
-  for (int slot = slot0; slot < slot1; ++slot) {
-    int held = idr[0];
+  // The row's plan ids, 64 per register (topk <= 64 * LS_DEC_ID_REGS).  (A vector:
+  // an array indexed in the lambda below would be kept in LDS.)
+  typedef int IdRegs __attribute__((ext_vector_type(LS_DEC_ID_REGS)));
+  IdRegs idr = -1;
+  int slot, slot1;  // the wave's next plan slot (DENSE: page) and the end of its share
+  if constexpr (DENSE) {
+    const int64_t n_vis = limit <= 0 ? 0 : limit < len_b ? (limit + 63) / 64 : n_pages;
+    const int share = (int)((n_vis + 4 * n_splits - 1) / (4 * n_splits));
+    slot = (4 * s + w) * share;
+    slot1 = (int)n_vis < slot + share ? (int)n_vis : slot + share;
+  } else {
+    const int32_t* idrow = topk_idx + ((int64_t)g * total_q + t) * topk;
 #pragma unroll
-    for (int k = 1; k < LS_DEC_ID_REGS; ++k)
-      if ((slot >> 6) == k) held = idr[k];
-    const int id = __builtin_amdgcn_readlane(held, slot & 63);
-    if (id < 0 || (int64_t)id >= n_pages || 64LL * id >= limit) continue;
-    // Skip a repeated id (the reference forms a page bitmask, so each page counts once).
-    bool dup = false;
+    for (int k = 0; k < LS_DEC_ID_REGS; ++k)
+      if (64 * k + lane < topk) idr[k] = idrow[64 * k + lane];
+    slot = (4 * s + w) * ppw;
+    slot1 = min(topk, slot + ppw);
+  }
+  // The page of the next valid slot (-1 at the end of the share).
+  auto next_page = [&]() -> int {
+    int found = -1;
+    while (found < 0 && slot < slot1) {
+      const int at = slot++;
+      if constexpr (DENSE) {
+        found = at;
+      } else {
+        const int held = at < 128 ? (at < 64 ? idr[0] : idr[1]) : (at < 192 ? idr[2] : idr[3]);
+        const int id = __builtin_amdgcn_readlane(held, at & 63);
+        if (id < 0 || (int64_t)id >= n_pages || 64LL * id >= limit) continue;
+        // Skip a repeated id (the reference forms a page bitmask, so each page counts once).
+        bool dup = false;
 #pragma unroll
-    for (int k = 0; k < LS_DEC_ID_REGS; ++k) dup |= __ballot(64 * k + lane < slot && idr[k] == id) != 0ull;
-    if (dup) continue;
-    const int64_t key0 = 64LL * id;
-    const int64_t nvis = min((int64_t)64, limit - key0);  // visible keys of this page (> 0)
-    // The page's K fragments and V rows are loaded together (keys past nvis as
-    // zeros).  K block kb = 2 c + nb, MFMA row R holds key 32 c + 8 (R / 4) + 4 nb + R % 4.
-    ls_u32x4 kf[4][4], vv[16];
+        for (int k = 0; k < LS_DEC_ID_REGS; ++k)
+          dup |= __ballot(64 * k + lane < at && idr[k] == id) != 0ull;
+        if (!dup) found = id;
+      }
+    }
+    return found;
+  };
+  // Visible keys of a page (> 0).  Rows past them are loaded as copies of the last
+  // visible one: their scores are masked, and their values replaced by zeros on
+  // the way to LDS.
+  auto visible = [&](int page) {
+    const int64_t n = limit - 64LL * page;
+    return n < 64 ? (int)n : 64;
+  };
+  ls_u32x4 kf[4][4], vv[16];
+  // K block kb = 2 c + nb, MFMA row R holds key 32 c + 8 (R / 4) + 4 nb + R % 4.
+  auto load_k = [&](int page) {
+    const int last = visible(page) - 1;
+    const uint16_t* kp = kseq + 64LL * page * crs + 8 * qg;
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) {
-      const int krow = 32 * (kb >> 1) + 8 * (r >> 2) + 4 * (kb & 1) + (r & 3);
-      const uint16_t* kp = kseq + (key0 + krow) * crs + 8 * qg;
+      const uint32_t krow = min(last, 32 * (kb >> 1) + 8 * (r >> 2) + 4 * (kb & 1) + (r & 3));
 #pragma unroll
-      for (int k4 = 0; k4 < 4; ++k4)
-        kf[kb][k4] = krow < nvis ? ls_load16(kp + 32 * k4) : ls_u32x4{0u, 0u, 0u, 0u};
+      for (int k4 = 0; k4 < 4; ++k4) kf[kb][k4] = ls_load16(kp + krow * (uint64_t)crs + 32 * k4);
     }
+  };
+  auto load_v = [&](int page) {
+    const int last = visible(page) - 1;
+    const uint16_t* vp = vseq + 64LL * page * crs + 8 * (lane & 15);
 #pragma unroll
     for (int it = 0; it < 16; ++it) {
-      const int ci = it * 64 + lane, kr = ci >> 4, c16 = ci & 15;
-      vv[it] = kr < nvis ? ls_load16(vseq + (key0 + kr) * crs + 8 * c16) : ls_u32x4{0u, 0u, 0u, 0u};
+      const uint32_t kr = min(last, 4 * it + (lane >> 4));
+      vv[it] = ls_load16(vp + kr * (uint64_t)crs);
     }
+  };
+  // One page whose K and V are in registers (or on their way), with the loads of
+  // the page after it.  The last page is its own copy of this code, so that the
+  // loads into the fragments are on every path of the loop (a conditional load
+  // would be copied, and so waited for, where the paths meet).
+  auto attend = [&](int page, int after, auto more) {
+    constexpr bool kMore = decltype(more)::value;
+    const int nvis = visible(page);
     float sv[16];
     float pm = -INFINITY;
 #pragma unroll
@@ -699,16 +749,21 @@ __global__ __launch_bounds__(256) void ls_decode_attn_kernel(
         pm = fmaxf(pm, v);
       }
     }
+    if constexpr (kMore) load_k(after);
     // V into the wave's LDS, rows of 128 values.
+    if (nvis < 64) {
+#pragma unroll
+      for (int it = 0; it < 16; ++it)
+        if (4 * it + (lane >> 4) >= nvis) vv[it] = ls_u32x4{0u, 0u, 0u, 0u};
+    }
 #pragma unroll
     for (int it = 0; it < 16; ++it) {
-      const int ci = it * 64 + lane, kr = ci >> 4, c16 = ci & 15;
-      uint32_t* dst = reinterpret_cast<uint32_t*>(sv_w + kr * LS_DEC_VPITCH + 16 * c16);
-      dst[0] = vv[it][0];
-      dst[1] = vv[it][1];
-      dst[2] = vv[it][2];
-      dst[3] = vv[it][3];
+      const int kr = 4 * it + (lane >> 4), c16 = lane & 15;
+      uint2* dst = reinterpret_cast<uint2*>(sv_w + kr * LS_DEC_VPITCH + 16 * c16);
+      dst[0] = make_uint2(vv[it][0], vv[it][1]);
+      dst[1] = make_uint2(vv[it][2], vv[it][3]);
     }
+    if constexpr (kMore) load_v(after);
     pm = fmaxf(pm, ls_shfl_xor(pm, 16));
     pm = fmaxf(pm, ls_shfl_xor(pm, 32));
     const float m_new = fmaxf(m_run, pm);  // finite: every page here has a visible key
@@ -751,6 +806,19 @@ __global__ __launch_bounds__(256) void ls_decode_attn_kernel(
       }
     }
     ls_dec_wave_sync();  // all reads of the page's V done before the next page overwrites it
+  };
+  int page = next_page();
+  if (page >= 0) {
+    load_k(page);
+    load_v(page);
+    __builtin_amdgcn_sched_barrier(0);  // both loads are under way before K is waited for
+    for (;;) {
+      const int after = next_page();
+      if (after < 0) break;
+      attend(page, after, std::true_type());
+      page = after;
+    }
+    attend(page, -1, std::false_type());
   }
   l_run += ls_shfl_xor(l_run, 16);
   l_run += ls_shfl_xor(l_run, 32);
@@ -1043,6 +1111,70 @@ extern "C" size_t ls_sparse_attn_kvcache_workspace_size(int64_t total_q, int32_t
                      LS_DEC_PART);
 }
 
+namespace {
+// Shared body of the planned (topk_idx, topk) and the dense (topk = 0) entry points.
+int kvcache_attn_run(const char* who, const void* q, int64_t q_row_stride,
+                     const int32_t* cu_seqlens_q, int64_t total_q, const void* k_cache,
+                     const void* v_cache, int64_t cache_batch_stride, int64_t cache_row_stride,
+                     const int32_t* cache_seqlens, int32_t batch, int32_t num_heads,
+                     int32_t num_kv_heads, int32_t head_dim, int32_t dtype,
+                     const int32_t* topk_idx, int32_t topk, bool dense, float softmax_scale,
+                     int32_t causal, int32_t n_splits, void* out, float* softmax_lse, void* ws,
+                     size_t ws_bytes, void* stream) {
+  LS_REQUIRE(batch > 0 && total_q >= 0 && num_kv_heads > 0 && num_heads % num_kv_heads == 0,
+             LS_ERR_INVALID, "%s: bad sizes", who);
+  const int gs = num_heads / num_kv_heads;
+  LS_REQUIRE(head_dim == 128 && gs >= 1 && gs <= 16, LS_ERR_UNSUPPORTED,
+             "%s: head_dim 128 and at most 16 query heads per KV head", who);
+  LS_REQUIRE(dtype == LS_BF16 || dtype == LS_F16, LS_ERR_UNSUPPORTED, "%s: bf16 or fp16", who);
+  LS_REQUIRE((dense || topk >= 1) && n_splits >= 1 && n_splits <= LS_DEC_MAX_SPLITS,
+             LS_ERR_INVALID, "%s: need topk >= 1 and 1 <= n_splits <= %d", who,
+             LS_DEC_MAX_SPLITS);
+  LS_REQUIRE(topk <= 64 * LS_DEC_ID_REGS, LS_ERR_UNSUPPORTED,
+             "%s: at most %d plan ids per row (got %d)", who, 64 * LS_DEC_ID_REGS, topk);
+  LS_REQUIRE(total_q <= 0x7fffffffLL && num_kv_heads <= 65535, LS_ERR_INVALID,
+             "%s: too many rows or heads", who);
+  LS_REQUIRE(q_row_stride % 8 == 0 && cache_row_stride % 8 == 0 && cache_batch_stride % 8 == 0,
+             LS_ERR_UNSUPPORTED, "%s: strides must be multiples of 8", who);
+  if (total_q == 0) return LS_OK;
+  LS_REQUIRE(q && k_cache && v_cache && cu_seqlens_q && cache_seqlens && (dense || topk_idx) &&
+                 out && ws,
+             LS_ERR_INVALID, "%s: null pointer", who);
+  LS_REQUIRE(ls_aligned16(q) && ls_aligned16(k_cache) && ls_aligned16(v_cache), LS_ERR_UNSUPPORTED,
+             "%s: tensors must be 16-byte aligned", who);
+  const size_t need = ls_sparse_attn_kvcache_workspace_size(total_q, num_kv_heads, n_splits);
+  LS_REQUIRE(ws_bytes >= need, LS_ERR_WORKSPACE, "%s: workspace %zu < %zu", who, ws_bytes, need);
+  // Four waves per split, ppw plan slots per wave.
+  const int ppw = (topk + 4 * n_splits - 1) / (4 * n_splits);
+  const int splits = dense ? n_splits : (topk + 4 * ppw - 1) / (4 * ppw);
+  hipStream_t s = (hipStream_t)stream;
+  const float scale_log2 = softmax_scale * 1.4426950408889634f;
+  float* part = (float*)ws;
+  const dim3 grid((unsigned)splits, (unsigned)total_q, num_kv_heads);
+  const dim3 cgrid((unsigned)total_q, num_kv_heads, gs);
+  auto attend = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, (const uint16_t*)q, q_row_stride,
+                       cu_seqlens_q, batch, total_q, (const uint16_t*)k_cache,
+                       (const uint16_t*)v_cache, cache_batch_stride, cache_row_stride,
+                       cache_seqlens, gs, head_dim, topk_idx, topk, ppw, splits, scale_log2,
+                       causal, part);
+    return ls_check_launch("ls_decode_attn_kernel");
+  };
+  int rc;
+  if (dtype == LS_BF16)
+    rc = dense ? attend(ls_decode_attn_kernel<LS_BF16, true>) : attend(ls_decode_attn_kernel<LS_BF16, false>);
+  else
+    rc = dense ? attend(ls_decode_attn_kernel<LS_F16, true>) : attend(ls_decode_attn_kernel<LS_F16, false>);
+  if (rc) return rc;
+  auto combine = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, cgrid, dim3(128), 0, s, part, total_q, gs, head_dim, splits,
+                       (uint16_t*)out, softmax_lse);
+  };
+  dtype == LS_BF16 ? combine(ls_decode_combine_kernel<LS_BF16>) : combine(ls_decode_combine_kernel<LS_F16>);
+  return ls_check_launch("ls_decode_combine_kernel");
+}
+}  // namespace
+
 extern "C" int ls_sparse_attn_kvcache(const void* q, int64_t q_row_stride,
                                       const int32_t* cu_seqlens_q, int64_t total_q,
                                       const void* k_cache, const void* v_cache,
@@ -1053,60 +1185,25 @@ extern "C" int ls_sparse_attn_kvcache(const void* q, int64_t q_row_stride,
                                       float softmax_scale, int32_t causal, int32_t n_splits,
                                       void* out, float* softmax_lse, void* ws, size_t ws_bytes,
                                       void* stream) {
-  LS_REQUIRE(batch > 0 && total_q >= 0 && num_kv_heads > 0 && num_heads % num_kv_heads == 0,
-             LS_ERR_INVALID, "ls_sparse_attn_kvcache: bad sizes");
-  const int gs = num_heads / num_kv_heads;
-  LS_REQUIRE(head_dim == 128 && gs >= 1 && gs <= 16, LS_ERR_UNSUPPORTED,
-             "ls_sparse_attn_kvcache: head_dim 128 and at most 16 query heads per KV head");
-  LS_REQUIRE(dtype == LS_BF16 || dtype == LS_F16, LS_ERR_UNSUPPORTED,
-             "ls_sparse_attn_kvcache: bf16 or fp16");
-  LS_REQUIRE(topk >= 1 && n_splits >= 1 && n_splits <= LS_DEC_MAX_SPLITS, LS_ERR_INVALID,
-             "ls_sparse_attn_kvcache: need topk >= 1 and 1 <= n_splits <= %d", LS_DEC_MAX_SPLITS);
-  LS_REQUIRE(topk <= 64 * LS_DEC_ID_REGS, LS_ERR_UNSUPPORTED,
-             "ls_sparse_attn_kvcache: at most %d plan ids per row (got %d)", 64 * LS_DEC_ID_REGS,
-             topk);
-  LS_REQUIRE(total_q <= 0x7fffffffLL && num_kv_heads <= 65535, LS_ERR_INVALID,
-             "ls_sparse_attn_kvcache: too many rows or heads");
-  LS_REQUIRE(q_row_stride % 8 == 0 && cache_row_stride % 8 == 0 && cache_batch_stride % 8 == 0,
-             LS_ERR_UNSUPPORTED, "ls_sparse_attn_kvcache: strides must be multiples of 8");
-  if (total_q == 0) return LS_OK;
-  LS_REQUIRE(q && k_cache && v_cache && cu_seqlens_q && cache_seqlens && topk_idx && out && ws,
-             LS_ERR_INVALID, "ls_sparse_attn_kvcache: null pointer");
-  LS_REQUIRE(ls_aligned16(q) && ls_aligned16(k_cache) && ls_aligned16(v_cache), LS_ERR_UNSUPPORTED,
-             "ls_sparse_attn_kvcache: tensors must be 16-byte aligned");
-  const size_t need = ls_sparse_attn_kvcache_workspace_size(total_q, num_kv_heads, n_splits);
-  LS_REQUIRE(ws_bytes >= need, LS_ERR_WORKSPACE, "ls_sparse_attn_kvcache: workspace %zu < %zu",
-             ws_bytes, need);
-  // Four waves per split, ppw plan slots per wave.
-  const int ppw = (topk + 4 * n_splits - 1) / (4 * n_splits);
-  const int splits = (topk + 4 * ppw - 1) / (4 * ppw);
-  hipStream_t s = (hipStream_t)stream;
-  const float scale_log2 = softmax_scale * 1.4426950408889634f;
-  float* part = (float*)ws;
-  const dim3 grid((unsigned)splits, (unsigned)total_q, num_kv_heads);
-  const dim3 cgrid((unsigned)total_q, num_kv_heads, gs);
-  if (dtype == LS_BF16) {
-    hipLaunchKernelGGL(ls_decode_attn_kernel<LS_BF16>, grid, dim3(256), 0, s, (const uint16_t*)q,
-                       q_row_stride, cu_seqlens_q, batch, total_q, (const uint16_t*)k_cache,
-                       (const uint16_t*)v_cache, cache_batch_stride, cache_row_stride,
-                       cache_seqlens, gs, head_dim, topk_idx, topk, ppw, splits, scale_log2,
-                       causal, part);
-    int rc = ls_check_launch("ls_decode_attn_kernel");
-    if (rc) return rc;
-    hipLaunchKernelGGL(ls_decode_combine_kernel<LS_BF16>, cgrid, dim3(128), 0, s, part, total_q,
-                       gs, head_dim, splits, (uint16_t*)out, softmax_lse);
-  } else {
-    hipLaunchKernelGGL(ls_decode_attn_kernel<LS_F16>, grid, dim3(256), 0, s, (const uint16_t*)q,
-                       q_row_stride, cu_seqlens_q, batch, total_q, (const uint16_t*)k_cache,
-                       (const uint16_t*)v_cache, cache_batch_stride, cache_row_stride,
-                       cache_seqlens, gs, head_dim, topk_idx, topk, ppw, splits, scale_log2,
-                       causal, part);
-    int rc = ls_check_launch("ls_decode_attn_kernel");
-    if (rc) return rc;
-    hipLaunchKernelGGL(ls_decode_combine_kernel<LS_F16>, cgrid, dim3(128), 0, s, part, total_q,
-                       gs, head_dim, splits, (uint16_t*)out, softmax_lse);
-  }
-  return ls_check_launch("ls_decode_combine_kernel");
+  return kvcache_attn_run("ls_sparse_attn_kvcache", q, q_row_stride, cu_seqlens_q, total_q, k_cache,
+                          v_cache, cache_batch_stride, cache_row_stride, cache_seqlens, batch,
+                          num_heads, num_kv_heads, head_dim, dtype, topk_idx, topk, false,
+                          softmax_scale, causal, n_splits, out, softmax_lse, ws, ws_bytes, stream);
+}
+
+extern "C" int ls_dense_attn_kvcache(const void* q, int64_t q_row_stride,
+                                     const int32_t* cu_seqlens_q, int64_t total_q,
+                                     const void* k_cache, const void* v_cache,
+                                     int64_t cache_batch_stride, int64_t cache_row_stride,
+                                     const int32_t* cache_seqlens, int32_t batch,
+                                     int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
+                                     int32_t dtype, float softmax_scale, int32_t causal,
+                                     int32_t n_splits, void* out, float* softmax_lse, void* ws,
+                                     size_t ws_bytes, void* stream) {
+  return kvcache_attn_run("ls_dense_attn_kvcache", q, q_row_stride, cu_seqlens_q, total_q, k_cache,
+                          v_cache, cache_batch_stride, cache_row_stride, cache_seqlens, batch,
+                          num_heads, num_kv_heads, head_dim, dtype, nullptr, 0, true,
+                          softmax_scale, causal, n_splits, out, softmax_lse, ws, ws_bytes, stream);
 }
 
 extern "C" size_t ls_stage1_scores_workspace_size(int64_t total_q, int32_t num_kv_heads,

@@ -17,7 +17,8 @@ from __future__ import annotations
 import torch
 
 from .ops.attention import infllmv2_attn_varlen_func
-from .ops.decode import kvcache_append, sparse_attention_kvcache, stage1_scores
+from .ops.decode import (dense_attention_kvcache, kvcache_append, sparse_attention_kvcache,
+                         stage1_scores)
 from .ops.nosa import max_pooling_1d_varlen
 
 __all__ = [
@@ -116,59 +117,18 @@ def infllmv2_attn_with_kvcache(q, k_cache, v_cache, k=None, v=None, rotary_cos=N
     cu_q = torch.arange(0, B * Sq + 1, Sq, dtype=torch.int32, device=dev)
     qr = q.reshape(B * Sq, H, D)
     splits = num_splits if num_splits > 0 else None
-    if topk_idx is None:  # every page of the longest sequence
-        out, lse = _dense_kvcache(qr, k_cache, v_cache, cache_seqlens, cu_q, max(lens), G,
-                                  bool(causal), softmax_scale, splits)
+    if topk_idx is None:  # every cached page
+        res = dense_attention_kvcache(qr, k_cache, v_cache, cache_seqlens, cu_q, max(lens),
+                                      causal=bool(causal), softmax_scale=softmax_scale,
+                                      n_splits=splits, return_lse=return_softmax_lse)
     else:
         res = sparse_attention_kvcache(qr, k_cache, v_cache, cache_seqlens, topk_idx, cu_q,
                                        causal=bool(causal), softmax_scale=softmax_scale,
                                        n_splits=splits, return_lse=return_softmax_lse)
-        out, lse = res if return_softmax_lse else (res, None)
+    out, lse = res if return_softmax_lse else (res, None)
     if return_softmax_lse:
         return out.view(B, Sq, H, D), lse.view(H, B, Sq).permute(1, 0, 2).contiguous()
     return out.view(B, Sq, H, D)
-
-
-_KV_MAX_IDS = 256  # ids per row of one ls_sparse_attn_kvcache call
-
-
-def _dense_kvcache(q, k_cache, v_cache, cache_seqlens, cu_q, max_len, G, causal, softmax_scale,
-                   n_splits):
-    """Attention over every cached page (``blockmask=None`` in the reference).
-
-    A row of one kvcache call holds at most 256 page ids, so a cache of more
-    pages is attended in groups of 256 pages whose partial results are merged
-    by their log-sum-exp: ``out = sum_i w_i out_i / sum_i w_i`` with ``w_i =
-    exp(lse_i - max lse)``; a group with no visible key (``lse = +inf``, ``out
-    = 0``) gets weight 0.  Each partial output is rounded to the activation
-    dtype before the merge, which is done in float32."""
-    n_pages = max(1, -(-max_len // 64))
-    total_q, H, _ = q.shape
-    dev = q.device
-    parts = []
-    for p0 in range(0, n_pages, _KV_MAX_IDS):
-        n = min(_KV_MAX_IDS, n_pages - p0)
-        ids = torch.arange(p0, p0 + n, dtype=torch.int32, device=dev).expand(G, total_q, n)
-        parts.append(sparse_attention_kvcache(q, k_cache, v_cache, cache_seqlens, ids, cu_q,
-                                              causal=causal, softmax_scale=softmax_scale,
-                                              n_splits=n_splits, return_lse=True))
-    if len(parts) == 1:
-        return parts[0]
-    lses = torch.stack([lse for _, lse in parts])               # [P, H, total_q]
-    lses = torch.where(torch.isinf(lses) & (lses > 0), torch.full_like(lses, float("-inf")), lses)
-    m = lses.amax(dim=0)
-    m_safe = torch.where(torch.isfinite(m), m, torch.zeros_like(m))
-    w = torch.exp(lses - m_safe)                                  # [P, H, total_q]
-    wsum = w.sum(dim=0)
-    acc = torch.zeros(total_q, H, q.shape[2], dtype=torch.float32, device=dev)
-    for (o, _), wi in zip(parts, w):
-        acc += o.float() * wi.t().unsqueeze(-1)
-    has = wsum > 0
-    inv = torch.where(has, 1.0 / torch.where(has, wsum, torch.ones_like(wsum)), torch.zeros_like(wsum))
-    out = (acc * inv.t().unsqueeze(-1)).to(q.dtype)
-    lse = torch.where(has, m_safe + torch.log(torch.where(has, wsum, torch.ones_like(wsum))),
-                      torch.full_like(wsum, float("inf")))
-    return out, lse
 
 
 max_pooling_1d = _not_provided("max_pooling_1d")

@@ -167,14 +167,34 @@ def sparse_attention_kvcache(q: torch.Tensor, k_cache: torch.Tensor, v_cache: to
     """``out [total_q, H, D]`` of the rows ``q [total_q, H, D]`` over the cache,
     restricted to each row's plan ``topk_idx [G, total_q, k]`` (and ``lse [H,
     total_q]`` float32 with ``return_lse``)."""
+    if topk_idx is None:
+        raise ValueError("q must be [total_q, H, D] and topk_idx [G, total_q, k]")
+    return _attend_cache(q, k_cache, v_cache, cache_seqlens, topk_idx, cu_seqlens_q, 0, causal,
+                         softmax_scale, n_splits, return_lse, out)
+
+
+def dense_attention_kvcache(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
+                            cache_seqlens: torch.Tensor, cu_seqlens_q: torch.Tensor, max_len: int,
+                            *, causal: bool = False, softmax_scale: float | None = None,
+                            n_splits: int | None = None, return_lse: bool = False):
+    """``sparse_attention_kvcache`` over every cached page; ``max_len`` is the longest
+    sequence's length."""
+    return _attend_cache(q, k_cache, v_cache, cache_seqlens, None, cu_seqlens_q,
+                         max(1, -(-int(max_len) // 64)), causal, softmax_scale, n_splits,
+                         return_lse, None)
+
+
+def _attend_cache(q, k_cache, v_cache, cache_seqlens, topk_idx, cu_seqlens_q, n_pages, causal,
+                  softmax_scale, n_splits, return_lse, out):
     _check_cache(k_cache, v_cache)
-    if q.ndim != 3 or topk_idx is None or topk_idx.ndim != 3:
+    if q.ndim != 3 or topk_idx is not None and topk_idx.ndim != 3:
         raise ValueError("q must be [total_q, H, D] and topk_idx [G, total_q, k]")
     total_q, H, D = q.shape
     B, cap, G, Dk = k_cache.shape
     if Dk != D or H % G or q.dtype != k_cache.dtype:
         raise ValueError("q and the cache must share head_dim and dtype, H divisible by G")
-    if topk_idx.shape[0] != G or topk_idx.shape[1] != total_q or not 1 <= topk_idx.shape[2] <= 256:
+    if topk_idx is not None and (topk_idx.shape[0] != G or topk_idx.shape[1] != total_q
+                                 or not 1 <= topk_idx.shape[2] <= 256):
         raise ValueError(f"topk_idx must be [{G}, {total_q}, k] with 1 <= k <= 256")
     if cache_seqlens.dtype != torch.int32 or cache_seqlens.numel() != B \
             or cu_seqlens_q.dtype != torch.int32 or cu_seqlens_q.numel() != B + 1:
@@ -182,15 +202,16 @@ def sparse_attention_kvcache(q: torch.Tensor, k_cache: torch.Tensor, v_cache: to
     if out is not None:
         _hip.check_out(out, (total_q, H, D), q.dtype, q.device)
     dev = _hip.require_gpu(q, k_cache, v_cache, cache_seqlens, topk_idx, cu_seqlens_q)
-    if topk_idx.dtype != torch.int32:
-        topk_idx = topk_idx.to(torch.int32)
-    topk_idx = topk_idx.contiguous()
+    if topk_idx is not None:
+        if topk_idx.dtype != torch.int32:
+            topk_idx = topk_idx.to(torch.int32)
+        topk_idx = topk_idx.contiguous()
+        n_pages = topk_idx.shape[2]
     q = q if (q.stride(2) == 1 and q.stride(1) == D) else q.contiguous()
-    K = topk_idx.shape[2]
     if n_splits is None:
         # Workgroups of four waves per (row, group): enough of them to cover the
         # device when there are few rows, at least one page per wave.
-        n_splits = max(1, min(-(-K // 4), -(-256 // max(1, total_q * G))))
+        n_splits = max(1, min(-(-n_pages // 4), -(-256 // max(1, total_q * G))))
     n_splits = max(1, min(int(n_splits), 64))
     if out is None:
         out = torch.empty((total_q, H, D), dtype=q.dtype, device=dev)
@@ -198,13 +219,16 @@ def sparse_attention_kvcache(q: torch.Tensor, k_cache: torch.Tensor, v_cache: to
     L = _hip.lib()
     ws = _hip.workspace(L.ls_sparse_attn_kvcache_workspace_size(total_q, G, n_splits), dev)
     scale = D ** -0.5 if softmax_scale is None else float(softmax_scale)
-    rc = L.ls_sparse_attn_kvcache(
-        q.data_ptr(), q.stride(0), cu_seqlens_q.contiguous().data_ptr(), total_q,
-        k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0), k_cache.stride(1),
-        cache_seqlens.contiguous().data_ptr(), B, H, G, D, _hip.dtype_code(q.dtype),
-        topk_idx.data_ptr(), K, scale, 1 if causal else 0, n_splits, out.data_ptr(),
-        _hip.ptr(lse), ws.data_ptr(), ws.numel(), _hip.stream_of(dev))
-    _hip.check(rc, "ls_sparse_attn_kvcache")
+    head = (q.data_ptr(), q.stride(0), cu_seqlens_q.contiguous().data_ptr(), total_q,
+            k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0), k_cache.stride(1),
+            cache_seqlens.contiguous().data_ptr(), B, H, G, D, _hip.dtype_code(q.dtype))
+    tail = (scale, 1 if causal else 0, n_splits, out.data_ptr(), _hip.ptr(lse), ws.data_ptr(),
+            ws.numel(), _hip.stream_of(dev))
+    if topk_idx is None:
+        _hip.check(L.ls_dense_attn_kvcache(*head, *tail), "ls_dense_attn_kvcache")
+    else:
+        _hip.check(L.ls_sparse_attn_kvcache(*head, topk_idx.data_ptr(), n_pages, *tail),
+                   "ls_sparse_attn_kvcache")
     return (out, lse) if return_lse else out
 
 

@@ -252,3 +252,10 @@ def test_fused_query_and_decode_entry_points_validate_before_any_launch():
     rc = lib.ls_sparse_attn_kvcache(None, 4096, None, 1, None, None, 0, 256, None, 1, 32, 2,
                                     128, B, None, 64, 0.088, 0, 65, None, None, None, 0, None)
     assert rc == _hip.LS_ERR_INVALID and b"n_splits" in lib.ls_last_error()
+    # ls_dense_attn_kvcache: too many splits, null tensors.
+    rc = lib.ls_dense_attn_kvcache(None, 4096, None, 1, None, None, 0, 256, None, 1, 32, 2,
+                                   128, B, 0.088, 0, 65, None, None, None, 0, None)
+    assert rc == _hip.LS_ERR_INVALID and b"n_splits" in lib.ls_last_error()
+    rc = lib.ls_dense_attn_kvcache(None, 4096, None, 1, None, None, 0, 256, None, 1, 32, 2,
+                                   128, B, 0.088, 0, 64, None, None, None, 0, None)
+    assert rc == _hip.LS_ERR_INVALID and b"null" in lib.ls_last_error()

@@ -359,6 +359,29 @@ def test_with_kvcache_dense_beyond_256_pages():
     torch.testing.assert_close(got_lse, want_lse.double(), rtol=0, atol=2e-3)
 
 
+@pytest.mark.parametrize("lens", [[1, 2], [64, 65], [63, 4097], [16384, 16385]])
+@pytest.mark.parametrize("splits", [0, 1, 64])
+def test_with_kvcache_dense_shares(lens, splits):
+    """The dense path's per-row shares of pages over splits and waves: rows of one
+    key, of whole pages and one key more, shares of none, one and several pages a
+    wave, and two causal rows a sequence whose visible pages differ."""
+    B, Sq, H = 2, 2 if min(lens) > 1 else 1, 32
+    k, v, _, kp, vp = _filled_cache(lens, -(-max(lens) // 64) * 64, seed=31)
+    g = torch.Generator().manual_seed(32)
+    q = torch.randn(B, Sq, H, D, generator=g).to(torch.bfloat16).to(DEV)
+    out, lse = infllmv2_attn_with_kvcache(q, k, v, cache_seqlens=_i32(lens), causal=True,
+                                          num_splits=splits, return_softmax_lse=True)
+    n_pages = -(-max(lens) // 64)
+    all_ids = torch.arange(n_pages, dtype=torch.int32).expand(G, B * Sq, n_pages).contiguous()
+    want, want_lse = oracle.sparse_attention(q.view(B * Sq, H, D).cpu(), kp, vp,
+                                             list(range(0, B * Sq + 1, Sq)), _cu(lens), all_ids,
+                                             causal=True)
+    ok, mx, mr = oracle.check_attention(out.view(B * Sq, H, D).cpu(), want)
+    assert ok, (mx, mr)
+    got_lse = lse.permute(1, 0, 2).reshape(H, B * Sq).cpu().double()
+    torch.testing.assert_close(got_lse, want_lse.double(), rtol=0, atol=2e-3)
+
+
 def test_model_decode_matches_prefill_when_every_page_is_kept():
     # With a budget above the page count both selectors keep every page, so a
     # decode step must give the logits of a prefill of the extended sequences.
