@@ -15,6 +15,7 @@
 // scores (infllmv2_attn_stage1, third_party/infllmv2/paper1.patch:1103-1302,
 // 2340-2362), and infllmv2_attn_with_kvcache with topk_idx
 // (paper1.patch:2511-2615).
+#include <algorithm>
 #include <type_traits>
 
 #include "ls_common.h"
@@ -32,93 +33,87 @@ __host__ __device__ __forceinline__ int64_t ls_n_windows(int64_t len, int ks, in
 }
 
 // ---------------------------------------------------------------------------
-// Append.  Thread (row, g, chunk of 8 channels) copies 16 bytes of K and of V
-// from the packed new rows to position cache_seqlens[b] + (row - cu_new[b]).
+// Append, one launch.  The first n_append workgroups copy the packed new rows:
+// thread (row, g, chunk of 8 channels) copies 16 bytes of K and of V to position
+// cache_seqlens[b] + (row - cu_new[b]).  The others form the compressed windows
+// the new tokens complete: win_blocks workgroups per sequence, a pair of threads
+// per (window, g, 8 channels), each summing one half of the window's rows
+// [w*stride, w*stride + ks) in float32 in token order (windows of two strides;
+// other geometries are summed by the first thread alone).  The halves are
+// added, the order of the prefill's half-window kernel, so a window formed here
+// is bit-identical to the one the prefill forms from the same keys.  Rows of
+// this call are read from the new keys rather than the cache, so the windows
+// need not wait for the copies, and each workgroup finds its sequence's windows
+// from its lengths, without a prefix sum over the batch: what were three launches
+// in a chain (copy 1.8, plan 1.4, windows 5.3 us for one sequence; 3.3, 4.4, 9.5
+// for sixteen) are one.
 // ---------------------------------------------------------------------------
+template <int DT>
 __global__ __launch_bounds__(256) void ls_cache_append_kernel(
-    uint16_t* __restrict__ kc_, uint16_t* __restrict__ vc_, int64_t cbs, int64_t crs,
+    uint16_t* kc_, uint16_t* __restrict__ vc_, int64_t cbs, int64_t crs,
     const int32_t* __restrict__ cache_seqlens, const uint16_t* __restrict__ kn,
     const uint16_t* __restrict__ vn, int64_t nrs, const int32_t* __restrict__ cu_new,
-    int64_t total_new, int batch, int G, int D) {
+    int64_t total_new, int batch, int G, int D, int64_t n_append, int win_blocks, int ks,
+    int stride, uint16_t* __restrict__ kcc, int64_t kbs, int64_t krs) {
   const int c8 = D / 8;
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int64_t per_row = (int64_t)G * c8;
-  const int64_t row = idx / per_row;
-  if (row >= total_new) return;
-  const int rem = (int)(idx - row * per_row);
-  const int g = rem / c8, c = rem - g * c8;
-  const int b = ls_find_segment(cu_new, batch, row);
-  const int64_t pos = (int64_t)cache_seqlens[b] + (row - cu_new[b]);
-  const int64_t src = row * nrs + (int64_t)g * D + 8 * c;
-  const int64_t dst = (int64_t)b * cbs + pos * crs + (int64_t)g * D + 8 * c;
-  *reinterpret_cast<ls_u32x4*>(kc_ + dst) = ls_load16(kn + src);
-  *reinterpret_cast<ls_u32x4*>(vc_ + dst) = ls_load16(vn + src);
-}
-
-// cu_win[b] = sum_{b' < b} (windows after the append - windows before it).
-__global__ void ls_cache_window_plan_kernel(const int32_t* __restrict__ cache_seqlens,
-                                            const int32_t* __restrict__ cu_new, int batch, int ks,
-                                            int stride, int32_t* __restrict__ cu_win) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  int32_t acc = 0;
-  cu_win[0] = 0;
-  for (int b = 0; b < batch; ++b) {
-    const int64_t l0 = cache_seqlens[b], l1 = l0 + (cu_new[b + 1] - cu_new[b]);
-    acc += (int32_t)(ls_n_windows(l1, ks, stride) - ls_n_windows(l0, ks, stride));
-    cu_win[b + 1] = acc;
+  const int64_t blk = blockIdx.x;
+  if (blk < n_append) {
+    const int64_t idx = blk * 256 + threadIdx.x;
+    const int64_t row = idx / per_row;
+    if (row >= total_new) return;
+    const int rem = (int)(idx - row * per_row);
+    const int g = rem / c8, c = rem - g * c8;
+    const int b = ls_find_segment(cu_new, batch, row);
+    const int64_t pos = (int64_t)cache_seqlens[b] + (row - cu_new[b]);
+    const int64_t src = row * nrs + (int64_t)g * D + 8 * c;
+    const int64_t dst = (int64_t)b * cbs + pos * crs + (int64_t)g * D + 8 * c;
+    *reinterpret_cast<ls_u32x4*>(kc_ + dst) = ls_load16(kn + src);
+    *reinterpret_cast<ls_u32x4*>(vc_ + dst) = ls_load16(vn + src);
+    return;
   }
-}
-
-// One thread per (new window, g, 8 channels): the window's mean over the
-// cache rows [w*stride, w*stride + ks), summed in float32 in token order.  For
-// windows of two strides the two halves are summed separately and added, the
-// order of the prefill's half-window kernel, so a window formed here is
-// bit-identical to the one the prefill forms from the same keys.
-template <int DT>
-__global__ __launch_bounds__(256) void ls_cache_compress_kernel(
-    const uint16_t* __restrict__ kcache, int64_t cbs, int64_t crs,
-    const int32_t* __restrict__ cache_seqlens, const int32_t* __restrict__ cu_win, int batch,
-    int G, int D, int ks, int stride, uint16_t* __restrict__ kcc, int64_t kbs, int64_t krs,
-    int64_t max_windows) {
-  const int c8 = D / 8;
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t per_win = (int64_t)G * c8;
-  const int64_t wi = idx / per_win;
-  if (wi >= max_windows || wi >= (int64_t)cu_win[batch]) return;
-  const int rem = (int)(idx - wi * per_win);
-  const int g = rem / c8, c = rem - g * c8;
-  const int b = ls_find_segment(cu_win, batch, wi);
-  const int64_t w = ls_n_windows(cache_seqlens[b], ks, stride) + (wi - cu_win[b]);
-  const uint16_t* src = kcache + (int64_t)b * cbs + (w * stride) * crs + (int64_t)g * D + 8 * c;
-  // Unrolled so that a block of row loads is in flight at once; the sums
-  // still run in token order.
-  auto add_rows = [&](int r0, int r1, float (&s)[8]) {
+  const int b = (int)((blk - n_append) / win_blocks);
+  const int64_t first = (blk - n_append) % win_blocks;
+  const int64_t l0 = cache_seqlens[b], n0 = cu_new[b];
+  const int64_t w0 = ls_n_windows(l0, ks, stride);
+  const int64_t n_win = ls_n_windows(l0 + (cu_new[b + 1] - n0), ks, stride) - w0;
+  const int half = threadIdx.x & 1;
+  const bool halves = ks == 2 * stride;
+  // Whole pairs leave the loop together (128 pairs per workgroup).
+  for (int64_t i = first * 128 + (threadIdx.x >> 1); i < n_win * per_row; i += 128LL * win_blocks) {
+    const int64_t wi = i / per_row;
+    const int rem = (int)(i - wi * per_row);
+    const int g = rem / c8, c = rem - g * c8;
+    const int64_t w = w0 + wi, p0 = w * stride;
+    const int64_t col = (int64_t)g * D + 8 * c;
+    const uint16_t* old_rows = kc_ + (int64_t)b * cbs + col;
+    const uint16_t* new_rows = kn + n0 * nrs + col;
+    const int r0 = halves ? half * stride : 0;
+    const int r1 = halves ? r0 + stride : (half ? 0 : ks);
+    float s[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s[e] = 0.f;
+    // Unrolled so that a block of row loads is in flight at once; the sums
+    // still run in token order.
 #pragma unroll 16
     for (int t = r0; t < r1; ++t) {
-      const ls_u32x4 a = ls_load16(src + (int64_t)t * crs);
+      const int64_t p = p0 + t;
+      const ls_u32x4 a = ls_load16(p < l0 ? old_rows + p * crs : new_rows + (p - l0) * nrs);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         s[2 * e] += LsElem<DT>::to_f((uint16_t)(a[e] & 0xffffu));
         s[2 * e + 1] += LsElem<DT>::to_f((uint16_t)(a[e] >> 16));
       }
     }
-  };
-  float acc[8], second[8];
+    const float n = (float)ks;
+    ls_u32x4 o;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) acc[e] = second[e] = 0.f;
-  if (ks == 2 * stride) {
-    add_rows(0, stride, acc);
-    add_rows(stride, ks, second);
-  } else {
-    add_rows(0, ks, acc);
+    for (int e = 0; e < 8; ++e) s[e] = (s[e] + ls_shfl_xor(s[e], 1)) / n;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      o[e] = ls_pack2(LsElem<DT>::from_f(s[2 * e]), LsElem<DT>::from_f(s[2 * e + 1]));
+    if (!half) *reinterpret_cast<ls_u32x4*>(kcc + (int64_t)b * kbs + w * krs + col) = o;
   }
-  const float n_win = (float)ks;
-  ls_u32x4 o;
-#pragma unroll
-  for (int e = 0; e < 4; ++e)
-    o[e] = ls_pack2(LsElem<DT>::from_f((acc[2 * e] + second[2 * e]) / n_win),
-                    LsElem<DT>::from_f((acc[2 * e + 1] + second[2 * e + 1]) / n_win));
-  *reinterpret_cast<ls_u32x4*>(kcc + (int64_t)b * kbs + w * krs + (int64_t)g * D + 8 * c) = o;
 }
 
 // ---------------------------------------------------------------------------
@@ -918,46 +913,40 @@ extern "C" int ls_kvcache_append(void* k_cache, void* v_cache, int64_t cache_bat
              LS_ERR_UNSUPPORTED, "ls_kvcache_append: head_dim and strides must be multiples of 8");
   LS_REQUIRE(cache_seqlens && cu_seqlens_new, LS_ERR_INVALID, "ls_kvcache_append: null lengths");
   hipStream_t s = (hipStream_t)stream;
+  int64_t n_append = 0, win_blocks = 0;
+  const int64_t per_row = (int64_t)num_kv_heads * (head_dim / 8);
   if (total_new > 0 && batch > 0) {
     LS_REQUIRE(k_cache && v_cache && k_new && v_new, LS_ERR_INVALID,
                "ls_kvcache_append: null tensor");
     LS_REQUIRE(ls_aligned16(k_cache) && ls_aligned16(v_cache) && ls_aligned16(k_new) &&
                    ls_aligned16(v_new),
                LS_ERR_UNSUPPORTED, "ls_kvcache_append: tensors must be 16-byte aligned");
-    const int64_t threads = total_new * num_kv_heads * (head_dim / 8);
-    hipLaunchKernelGGL(ls_cache_append_kernel, dim3((unsigned)((threads + 255) / 256)),
-                       dim3(256), 0, s, (uint16_t*)k_cache, (uint16_t*)v_cache,
-                       cache_batch_stride, cache_row_stride, cache_seqlens,
-                       (const uint16_t*)k_new, (const uint16_t*)v_new, new_row_stride,
-                       cu_seqlens_new, total_new, batch, num_kv_heads, head_dim);
-    int rc = ls_check_launch("ls_cache_append_kernel");
-    if (rc) return rc;
+    n_append = (total_new * per_row + 255) / 256;
   }
-  if (!kc_cache || batch == 0) return LS_OK;
-  LS_REQUIRE(kernel_size > 0 && kernel_stride > 0, LS_ERR_INVALID,
-             "ls_kvcache_append: kernel_size and kernel_stride must be positive");
-  LS_REQUIRE(cu_windows, LS_ERR_INVALID, "ls_kvcache_append: null cu_windows");
-  LS_REQUIRE(ls_aligned16(kc_cache) && kc_row_stride % 8 == 0 && kc_batch_stride % 8 == 0,
-             LS_ERR_UNSUPPORTED, "ls_kvcache_append: compressed cache must be 16-byte aligned");
-  hipLaunchKernelGGL(ls_cache_window_plan_kernel, dim3(1), dim3(64), 0, s, cache_seqlens,
-                     cu_seqlens_new, batch, kernel_size, kernel_stride, cu_windows);
-  int rc = ls_check_launch("ls_cache_window_plan_kernel");
-  if (rc || max_new_windows <= 0) return rc;
-  const int64_t threads = max_new_windows * num_kv_heads * (head_dim / 8);
-  const dim3 grid((unsigned)((threads + 255) / 256));
-  if (dtype == LS_BF16)
-    hipLaunchKernelGGL(ls_cache_compress_kernel<LS_BF16>, grid, dim3(256), 0, s,
-                       (const uint16_t*)k_cache, cache_batch_stride, cache_row_stride,
-                       cache_seqlens, cu_windows, batch, num_kv_heads, head_dim, kernel_size,
-                       kernel_stride, (uint16_t*)kc_cache, kc_batch_stride, kc_row_stride,
-                       max_new_windows);
-  else
-    hipLaunchKernelGGL(ls_cache_compress_kernel<LS_F16>, grid, dim3(256), 0, s,
-                       (const uint16_t*)k_cache, cache_batch_stride, cache_row_stride,
-                       cache_seqlens, cu_windows, batch, num_kv_heads, head_dim, kernel_size,
-                       kernel_stride, (uint16_t*)kc_cache, kc_batch_stride, kc_row_stride,
-                       max_new_windows);
-  return ls_check_launch("ls_cache_compress_kernel");
+  if (kc_cache && batch > 0) {
+    LS_REQUIRE(kernel_size > 0 && kernel_stride > 0, LS_ERR_INVALID,
+               "ls_kvcache_append: kernel_size and kernel_stride must be positive");
+    LS_REQUIRE(cu_windows, LS_ERR_INVALID, "ls_kvcache_append: null cu_windows");
+    LS_REQUIRE(ls_aligned16(kc_cache) && kc_row_stride % 8 == 0 && kc_batch_stride % 8 == 0,
+               LS_ERR_UNSUPPORTED, "ls_kvcache_append: compressed cache must be 16-byte aligned");
+    // Enough workgroups for the whole batch's windows in one sequence, as far as
+    // the launch stays small (a workgroup then loops over more of its windows).
+    if (max_new_windows > 0 && n_append > 0)
+      win_blocks = std::min<int64_t>((max_new_windows * per_row + 127) / 128,
+                                     std::max<int64_t>(1, 4096 / batch));
+  }
+  const int64_t blocks = n_append + win_blocks * batch;
+  if (blocks == 0) return LS_OK;
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, s, (uint16_t*)k_cache,
+                       (uint16_t*)v_cache, cache_batch_stride, cache_row_stride, cache_seqlens,
+                       (const uint16_t*)k_new, (const uint16_t*)v_new, new_row_stride,
+                       cu_seqlens_new, total_new, batch, num_kv_heads, head_dim, n_append,
+                       (int)std::max<int64_t>(1, win_blocks), kernel_size, kernel_stride,
+                       (uint16_t*)kc_cache, kc_batch_stride, kc_row_stride);
+  };
+  dtype == LS_BF16 ? launch(ls_cache_append_kernel<LS_BF16>) : launch(ls_cache_append_kernel<LS_F16>);
+  return ls_check_launch("ls_cache_append_kernel");
 }
 
 namespace {

@@ -359,6 +359,37 @@ def test_with_kvcache_dense_beyond_256_pages():
     torch.testing.assert_close(got_lse, want_lse.double(), rtol=0, atol=2e-3)
 
 
+@pytest.mark.parametrize("ks,stride", [(32, 16), (48, 16), (16, 16), (7, 3)])
+@pytest.mark.parametrize("lens,n_new", [([0, 31, 100], [40, 1, 0]), ([47, 5], [1, 1]),
+                                        ([1000, 0, 3, 16], [700, 15, 2000, 16])])
+def test_append_window_geometries(ks, stride, lens, n_new):
+    """Windows over old and new rows, of two halves and not, sequences without new
+    rows or without a window among them: each new window is the mean of its rows to
+    one rounding, and nothing else of the compressed cache changes."""
+    B, cap = len(lens), 2048
+    g = torch.Generator().manual_seed(41)
+    rnd = lambda *shape: torch.randn(*shape, generator=g).to(torch.bfloat16).to(DEV)  # noqa: E731
+    k, v = rnd(B, cap, G, D), rnd(B, cap, G, D)
+    kn, vn = rnd(sum(n_new), G, D), rnd(sum(n_new), G, D)
+    kc = torch.full((B, cap, G, D), 7.0, dtype=torch.bfloat16, device=DEV)
+    cu = _cu(n_new)
+    want_k = k.clone()
+    kvcache_append(k, v, _i32(lens), kn, vn, _i32(cu), kc_cache=kc, kernel_size=ks,
+                   kernel_stride=stride)
+    for b in range(B):
+        lo, hi = lens[b], lens[b] + n_new[b]
+        want_k[b, lo:hi] = kn[cu[b]:cu[b + 1]]
+        assert torch.equal(v[b, lo:hi], vn[cu[b]:cu[b + 1]])
+        w0, w1 = ((n - ks) // stride + 1 if n >= ks else 0 for n in (lo, hi))
+        assert bool((kc[b, :w0] == 7).all()) and bool((kc[b, w1:] == 7).all())
+        if w1 > w0:
+            want = want_k[b, :hi].double().unfold(0, ks, stride).mean(-1)[w0:w1]
+            # One bf16 rounding of a float32 mean (half a step, and the sum's error).
+            assert bool(((kc[b, w0:w1].double() - want).abs()
+                         <= 0.51 * oracle.output_step(want, torch.bfloat16) + 1e-6).all())
+    assert torch.equal(k, want_k)
+
+
 @pytest.mark.parametrize("lens", [[1, 2], [64, 65], [63, 4097], [16384, 16385]])
 @pytest.mark.parametrize("splits", [0, 1, 64])
 def test_with_kvcache_dense_shares(lens, splits):
