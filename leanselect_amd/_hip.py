@@ -132,9 +132,12 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_DTYPE_CODES = {torch.float32: LS_F32, torch.bfloat16: LS_BF16, torch.float16: LS_F16}
+
+
 def dtype_code(dtype: torch.dtype) -> int:
     try:
-        return {torch.float32: LS_F32, torch.bfloat16: LS_BF16, torch.float16: LS_F16}[dtype]
+        return _DTYPE_CODES[dtype]
     except KeyError:
         raise ValueError(f"unsupported dtype {dtype}; expected float32, bfloat16 or float16")
 
@@ -266,7 +269,8 @@ def poll_attn_status() -> None:
 
 
 def stream_of(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    # The raw handle, without building a Stream object on every launch.
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def workspace(nbytes: int, device: torch.device) -> torch.Tensor:

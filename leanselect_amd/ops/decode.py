@@ -33,7 +33,7 @@ def n_windows(length: int, kernel_size: int = 32, kernel_stride: int = 16) -> in
 def _lengths(t: torch.Tensor, host, name: str) -> list[int]:
     if t.dtype != torch.int32 or t.ndim != 1:
         raise ValueError(f"{name} must be a 1-D int32 tensor")
-    return [int(x) for x in (host if host is not None else t.tolist())]
+    return list(map(int, host)) if host is not None else t.tolist()
 
 
 def _check_cache(k_cache: torch.Tensor, v_cache: torch.Tensor) -> None:
