@@ -303,10 +303,11 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
   // ---- per-row state: Q^T fragments (B operand), softmax stats, O^T ----
   // (the Q loads are issued first; they land while the page list is built)
   ls_u32x4 qf[TPW][4];
-  // thr: the score (raw, or in base-2 units with a bias) above which a key would
-  // exceed the running maximum m = thr * scale_log2 - 8 (thr - 8 with a bias) by
-  // more than 2^8; m itself is not kept.
-  float l_run[TPW], thr[TPW];
+  // m_run: running maximum in base-2 units (score * scale_log2).  The score above
+  // which a key would exceed it by more than 2^8 is formed from it for each chunk:
+  // the maximum formed from that score instead would be rounded once more, and so
+  // would the lse.
+  float m_run[TPW], l_run[TPW];
   int jmax_r[TPW];
   ls_f32x4 o[TPW][8];
 #pragma unroll
@@ -320,7 +321,7 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
       if (!head_ok) qf[j][ks] = ls_u32x4{0u, 0u, 0u, 0u};
     }
     l_run[j] = 0.f;
-    thr[j] = -INFINITY;
+    m_run[j] = -INFINITY;
     // Wave-uniform, so each chunk's row mask below is scalar work.
     jmax_r[j] = __builtin_amdgcn_readfirstlane(row < n_rows ? (int)row_jmax(row) : -1);
 #pragma unroll
@@ -377,7 +378,6 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
     return __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(x)));
   };
   const float inv_scale_log2 = uniform_f(1.f / scale_log2);
-  auto run_max = [&](float t) { return BIAS ? t - 8.f : fmaf(t, scale_log2, -8.f); };
   // Page order.  Where the rows share many pages (at least
   // LS_ATT_SHARE_STRIDED / 10 plan ids per union page) the pages are visited in
   // a strided order (ascending page i goes to slot i * stride mod n_union, a
@@ -560,8 +560,8 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
         for (int i = 0; i < 8; ++i)
           if (i > lim) sv[i] = -INFINITY;
       }
-      // With a bias the scores are taken to base-2 units here (thr and the
-      // maxima below are then all in those units).
+      // With a bias the scores are taken to base-2 units here (the maxima and
+      // the threshold below are then in those units).
       if constexpr (BIAS) {
         const float* bp = s_bias + (ui % LS_ATT_STAGES) * 64 + 32 * c + 8 * q;
         const ls_f32x4 cbv0 = *reinterpret_cast<const ls_f32x4*>(bp);
@@ -580,22 +580,21 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
                                fmaxf(fmaxf(sv[3], sv[4]), sv[5]));
       // Rescale only when some head's max grows by more than 2^8 (or when the
       // page's V scale leaves too little fp16 headroom for P up to 2^8).
-      if (__builtin_expect((__ballot(lmax > thr[j]) | ve_mask) != 0ull, 0)) {
+      const float thr = BIAS ? m_run[j] + 8.f : (m_run[j] + 8.f) * inv_scale_log2;
+      if (__builtin_expect((__ballot(lmax > thr) | ve_mask) != 0ull, 0)) {
         float cm = lmax;
         cm = fmaxf(cm, ls_shfl_xor(cm, 16));
         cm = fmaxf(cm, ls_shfl_xor(cm, 32));
-        const float m_old = run_max(thr[j]);
-        const float m_new = fmaxf(m_old, BIAS ? cm : cm * scale_log2);
-        thr[j] = BIAS ? m_new + 8.f : (m_new + 8.f) * inv_scale_log2;
-        const float alpha = __builtin_amdgcn_exp2f(m_old - run_max(thr[j]));
+        const float m_new = fmaxf(m_run[j], BIAS ? cm : cm * scale_log2);
+        const float alpha = __builtin_amdgcn_exp2f(m_run[j] - m_new);
+        m_run[j] = m_new;
         l_run[j] *= alpha;
 #pragma unroll
         for (int db = 0; db < 8; ++db) o[j][db] *= alpha;
       }
       // P' = P * 2^e (the page's V scale moved onto P, exact): one exp each;
       // the row sum adds the fp16 P' that the MFMA uses, scaled back by 2^-e.
-      const float bias = BIAS ? (float)(v_e + 8) - thr[j]
-                              : fmaf(-scale_log2, thr[j], (float)(v_e + 8));
+      const float bias = (float)v_e - m_run[j];
       ls_u32x4 pf;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -709,7 +708,7 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
     }
     if (lse && q == 0)
       lse[((int64_t)g * gs + head) * total_q + t] =
-          l_tot > 0.f ? run_max(thr[j]) * 0.69314718055994531f + __logf(l_tot) : INFINITY;
+          l_tot > 0.f ? m_run[j] * 0.69314718055994531f + __logf(l_tot) : INFINITY;
   }
 }
 

@@ -265,6 +265,32 @@ def test_attention_tile_sizes_and_tile_deal(lens, biased):
     assert bool(torch.isfinite(out).all())
 
 
+@pytest.mark.parametrize("n", [1500, 4200])
+@pytest.mark.parametrize("amp", [1, 8])
+def test_attention_lse_of_one_key_is_its_score(n, amp):
+    """A row that sees one key has that key's scaled score as its log-sum-exp.
+    Integer queries and keys make the score exact in float32, and the scale is a
+    power of two, so the float32 path rounds twice (the product with log2 e, the
+    one with ln 2, 2^-24 each) on top of the two constants' own errors (together
+    below 2^-25): 2.5 x 2^-24 of the value."""
+    G, H, D = 2, 32, 128
+    g = torch.Generator().manual_seed(51)
+    ints = lambda *shape: torch.randint(-amp, amp + 1, shape, generator=g)  # noqa: E731
+    q, k, v = ints(n, H, D), ints(n, G, D), ints(n, G, D)
+    t16 = lambda x: x.to(torch.bfloat16).to(DEV)  # noqa: E731
+    ids = (torch.arange(n, dtype=torch.int32) // 64)[None, :, None].expand(G, n, 1).contiguous()
+    cu = torch.tensor([0, n], dtype=torch.int32, device=DEV)
+    out, lse = sparse_attention(t16(q), t16(k), t16(v), cu, cu, n, n, ids.to(DEV),
+                                softmax_scale=0.125, return_lse=True)
+    rows = torch.arange(0, n, 64)  # the first row of a page sees that page's first key only
+    want = (q[rows].view(-1, G, H // G, D) * k[rows][:, :, None]).sum(-1).double() * 0.125
+    want = want.reshape(-1, H).t()
+    got = lse.cpu()[:, rows].double()
+    assert bool(((got - want).abs() <= 2.5 * 2.0 ** -24 * want.abs()).all())
+    assert torch.equal(out.cpu()[rows].float().view(-1, G, H // G, D),
+                       v[rows].float()[:, :, None].expand(-1, G, H // G, D))
+
+
 def test_attention_messy_ids_duplicates_unsorted_out_of_range():
     case, ids = _attention_case(lens=(1500,), seed=7)
     g = torch.Generator(device="cpu").manual_seed(0)
