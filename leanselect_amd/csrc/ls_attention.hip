@@ -6,7 +6,7 @@
 // keys are those of the valid ids in topk_idx[g, t, :] (each page once) with
 // j <= t + len_k - len_q when causal; all H/G heads of the group share the plan.
 //
-// Design (one workgroup per 24 query rows of one KV group and 16-head tile):
+// Design (one workgroup per 8, 12 or 24 query rows of one KV group and 16-head tile):
 //   * the plan rows are turned into an ascending, duplicate-free page list
 //     through an LDS table of row masks (ids past the causal frontier are dropped);
 //   * S^T = K . Q^T on v_mfma_f32_16x16x32: keys are MFMA rows, the 16 heads of
@@ -71,9 +71,9 @@ __global__ void ls_attn_status_clear_kernel(int32_t* __restrict__ status) {
 }
 
 // ---------------------------------------------------------------------------
-// Tile kernel: one workgroup = 8 x TPW consecutive query rows of one sequence
-// and one KV group for 16 of its query heads (8 waves x TPW rows, two waves per
-// SIMD; the launcher picks TPW).  The rows' page plans are OR-ed into a union page list;
+// Tile kernel: one workgroup = 8, 12 or 24 consecutive query rows of one sequence
+// and one KV group for 16 of its query heads (8 waves of up to TPW rows, two waves
+// per SIMD; the launcher picks TPW).  The rows' page plans are OR-ed into a union page list;
 // each union page of staged K and V^T is streamed once into a 4-stage LDS ring
 // with direct global->LDS loads, and every row that selected the page runs its
 // MFMAs on it.  Rows that did not select a page skip it (no masked-out work).
@@ -97,15 +97,36 @@ __global__ void ls_attn_status_clear_kernel(int32_t* __restrict__ status) {
 #endif
 #define LS_ATT_UNION_CAP 4096                // union pages of a tile (ready tokens in the workspace)
 
-// Tile geometry for TPW rows per wave: rows per tile, the most ids per row it
-// accepts (so that its union fits LS_ATT_UNION_CAP) and the union bound.
+// Tile geometry for at most TPW rows per wave: rows per tile, each wave's rows,
+// the most ids per row it accepts (so that its union fits LS_ATT_UNION_CAP) and
+// the union bound.  Tiles have 8, 12 or 24 rows: with TPW = 2 the first half of the
+// waves has two rows and the other half one, three on every SIMD (waves w and w + 4
+// share one).
+//
+// A row's pages are visited in the order that the plans of the 24 rows around it
+// give (rows 24 i .. 24 i + 23 of the sequence, the group of rows, which holds
+// whole tiles of each height).  So a row's sums, and with them its output, are bit
+// for bit the same whichever height the launcher takes: they don't depend on what
+// else is packed into the call.  (Tiles of 16 rows would straddle two groups, with
+// both groups' orders to form and pages copied for each: 197 us for 4096 rows,
+// where 24-row tiles take 205.)
+#define LS_ATT_GROUP 24
 template <int TPW>
 struct LsAttTile {
-  static constexpr int kTile = LS_ATT_WAVES * TPW;
+  static constexpr int kTile = TPW == 2 ? 12 : LS_ATT_WAVES * TPW;
   static constexpr int kMaxTake =
       LS_ATTN_MAX_TAKE < LS_ATT_UNION_CAP / kTile ? LS_ATTN_MAX_TAKE : LS_ATT_UNION_CAP / kTile;
   static constexpr int kMaxUnion = kTile * kMaxTake;
-  static_assert(kTile <= 32, "row masks are 32-bit");
+  __host__ __device__ static constexpr int rows(int w) {
+    return TPW == 2 && w >= LS_ATT_WAVES / 2 ? 1 : TPW;
+  }
+  __host__ __device__ static constexpr int row0(int w) {
+    return TPW == 2 && w >= LS_ATT_WAVES / 2 ? w + LS_ATT_WAVES / 2 : w * TPW;
+  }
+  static_assert(LS_ATT_WAVES == 8 && row0(LS_ATT_WAVES - 1) + rows(LS_ATT_WAVES - 1) == kTile,
+                "the waves' rows make up the tile");
+  static_assert(kTile <= LS_ATT_GROUP && LS_ATT_GROUP % kTile == 0 && LS_ATT_GROUP <= 32,
+                "a group holds whole tiles, and its row masks are 32-bit");
   static_assert(kMaxUnion <= LS_ATT_UNION_CAP, "one ready token per union page");
 };
 
@@ -236,12 +257,16 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
   constexpr int TILE = LsAttTile<TPW>::kTile;
   constexpr int MAX_UNION = LsAttTile<TPW>::kMaxUnion;
   constexpr int MAX_VISITS = TPW * LsAttTile<TPW>::kMaxTake;  // pages of one wave
-  constexpr uint32_t ROWS_MASK = (1u << TPW) - 1u;
-  // The setup tables (rows per page, rows per union page) are only needed
-  // before streaming starts and share their LDS with the ring.
+  constexpr int GROUP = LS_ATT_GROUP, GROUP_RPW = GROUP / LS_ATT_WAVES;
+  constexpr int MAX_ORDER = GROUP * LsAttTile<TPW>::kMaxTake;  // pages of a group
+  constexpr uint32_t TILE_MASK = (1u << TILE) - 1u;
+  // The setup tables (rows per page, the group's pages in visit order) are only
+  // needed before streaming starts and share their LDS with the ring.
   __shared__ __align__(16) uint8_t s_ring[LS_ATT_STAGES * LS_ATT_STAGE_BYTES];
-  uint32_t* s_rows = reinterpret_cast<uint32_t*>(s_ring);  // [page]: mask of the tile rows on it
-  uint32_t* s_umeta = s_rows + LS_ATTN_MAX_PAGES;          // [union page]: the same mask
+  uint32_t* s_rows = reinterpret_cast<uint32_t*>(s_ring);  // [page]: mask of the group rows on it
+  uint32_t* s_omask = s_rows + LS_ATTN_MAX_PAGES;          // [place in the order]: the same mask
+  uint16_t* s_opage = reinterpret_cast<uint16_t*>(s_omask + MAX_ORDER);  // and the page
+  // The tile's own pages, the union, in that order.
   __shared__ uint16_t s_upage[MAX_UNION];
   __shared__ uint8_t s_uneed[MAX_UNION];  // waves with a row on the page
   // The pages of each wave in the order it visits them: page | its rows on it
@@ -255,15 +280,18 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
   __shared__ uint32_t s_next, s_done[LS_ATT_STAGES];
   __shared__ __align__(8) uint32_t s_rdy[LS_ATT_STAGES][2];
   __shared__ __align__(16) float s_bias[BIAS ? LS_ATT_STAGES * 64 : 4];
-  static_assert((LS_ATTN_MAX_PAGES + MAX_UNION) * 4 <= LS_ATT_STAGES * LS_ATT_STAGE_BYTES,
+  static_assert(LS_ATTN_MAX_PAGES * 4 + MAX_ORDER * 6 <= LS_ATT_STAGES * LS_ATT_STAGE_BYTES,
                 "the setup tables must fit in the ring");
-  static_assert(TILE <= 32, "row masks are 32-bit");
+  static_assert(GROUP % LS_ATT_WAVES == 0, "each wave takes part in the setup alike");
   static_assert(LS_ATTN_MAX_PAGES <= 1 << 13 && TPW <= 3 && MAX_UNION <= 1 << 16,
                 "fields of a visit entry");
 
   const int tid = LS_TID;
   const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, q = lane >> 4;
+  // This wave's rows of the tile: n_mine from row w0 on.
+  const int w0 = LsAttTile<TPW>::row0(w), n_mine = LsAttTile<TPW>::rows(w);
+  const uint32_t rows_mask = (1u << n_mine) - 1u;
 
   // XCD-aware tile order.  Consecutive workgroups land on different XCDs
   // (workgroup x runs on XCD x % 8).  Each XCD takes runs of `run` consecutive
@@ -290,15 +318,19 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
   const int lk = cu_k[b + 1] - cu_k[b];
   const int64_t vbase = 64LL * pg_off[b];
   const int64_t tr0 = t0 - cu_q[b];
-  // Keys visible to row i of the tile: j <= jmax(i) (the last row sees the most).
+  // The tile's group: rows gr0 .. gr0 + n_grp - 1 of the sequence, the tile's from `off` on.
+  const int64_t gr0 = tr0 / GROUP * GROUP;
+  const int off = (int)(tr0 - gr0);
+  const int n_grp = (int)min((int64_t)GROUP, (int64_t)lq - gr0);
+  // Keys visible to row i of the group: j <= jmax(i) (the last row sees the most).
   auto row_jmax = [&](int i) -> int64_t {
     int64_t jm = lk - 1;
-    if (causal) jm = min(jm, tr0 + i + (int64_t)(lk - lq));
+    if (causal) jm = min(jm, gr0 + i + (int64_t)(lk - lq));
     return jm;
   };
-  const int64_t tile_jmax = row_jmax(n_rows - 1);
+  const int64_t group_jmax = row_jmax(n_grp - 1);
   const int last_page =
-      tile_jmax >= 0 ? (int)min(tile_jmax / 64, (int64_t)LS_ATTN_MAX_PAGES - 1) : -1;
+      group_jmax >= 0 ? (int)min(group_jmax / 64, (int64_t)LS_ATTN_MAX_PAGES - 1) : -1;
 
   // ---- per-row state: Q^T fragments (B operand), softmax stats, O^T ----
   // (the Q loads are issued first; they land while the page list is built)
@@ -312,7 +344,7 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
   ls_f32x4 o[TPW][8];
 #pragma unroll
   for (int j = 0; j < TPW; ++j) {
-    const int row = w * TPW + j;
+    const int row = w0 + j;
     const int64_t t = t0 + min(row, n_rows - 1);
     const uint16_t* qrow = qg + t * q_rs + ((int64_t)g * gs + (head_ok ? head : 0)) * D + 8 * q;
 #pragma unroll
@@ -323,11 +355,11 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
     l_run[j] = 0.f;
     m_run[j] = -INFINITY;
     // Wave-uniform, so each chunk's row mask below is scalar work.
-    jmax_r[j] = __builtin_amdgcn_readfirstlane(row < n_rows ? (int)row_jmax(row) : -1);
+    jmax_r[j] = __builtin_amdgcn_readfirstlane(j < n_mine && row < n_rows ? (int)row_jmax(off + row) : -1);
 #pragma unroll
     for (int db = 0; db < 8; ++db) o[j][db] = ls_f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  // ---- the tile's pages: rows per page, then their ascending union ----
+  // ---- the group's pages: rows per page, then their order, then the tile's among them ----
   // Every step works on 64 pages or ids per wave at a time: the tile's setup
   // is exposed (one workgroup fills a CU's LDS), so it must not loop serially
   // over a word's bits or a thread's pages.
@@ -339,12 +371,13 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
   if (tid == 0) s_next = LS_ATT_STAGES;  // pages 0..3 are copied at the start
   __syncthreads();
   if (last_page >= 0) {
-    const int32_t* ids = topk_idx + ((int64_t)g * total_q + t0) * take;
+    const int32_t* ids = topk_idx + ((int64_t)g * total_q + cu_q[b] + gr0) * take;
 #pragma unroll
-    for (int j = 0; j < TPW; ++j) {
-      const int row = w * TPW + j;
-      const int pmax = jmax_r[j] >= 0 ? min(jmax_r[j] / 64, last_page) : -1;
-      if (row < n_rows)
+    for (int j = 0; j < GROUP_RPW; ++j) {
+      const int row = w * GROUP_RPW + j;
+      const int jm = __builtin_amdgcn_readfirstlane((int)row_jmax(row));
+      const int pmax = jm >= 0 ? min(jm / 64, last_page) : -1;
+      if (row < n_grp)
         for (int i = lane; i < take; i += 64) {
           const int p = ids[(int64_t)row * take + i];
           if (p >= 0 && p <= pmax) atomicOr(&s_rows[p], 1u << row);
@@ -362,15 +395,15 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
   }
   if (lane == 0) s_wsum[w] = wave_pages;
   __syncthreads();
-  int pos0 = 0, n_union = 0;
+  int pos0 = 0, n_order = 0;
 #pragma unroll
   for (int i = 0; i < LS_ATT_WAVES; ++i) {
     const int c = s_wsum[i];
     pos0 += i < w ? c : 0;
-    n_union += c;
+    n_order += c;
   }
   pos0 = __builtin_amdgcn_readfirstlane(pos0);
-  n_union = __builtin_amdgcn_readfirstlane(n_union);
+  n_order = __builtin_amdgcn_readfirstlane(n_order);
   const int32_t* vexp_seq = vexp + (int64_t)g * n_pages_ws + pg_off[b];
   // Wave-uniform floats are kept in scalar registers: with three rows of O and Q,
   // the chunk's K and V^T fragments and a row's scores no vector register is spare.
@@ -378,21 +411,21 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
     return __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(x)));
   };
   const float inv_scale_log2 = uniform_f(1.f / scale_log2);
-  // Page order.  Where the rows share many pages (at least
-  // LS_ATT_SHARE_STRIDED / 10 plan ids per union page) the pages are visited in
-  // a strided order (ascending page i goes to slot i * stride mod n_union, a
-  // bijection for stride coprime to n_union): neighbouring pages tend to be
+  // Page order.  Where the group's rows share many pages (at least
+  // LS_ATT_SHARE_STRIDED / 10 plan ids per page) the pages are visited in
+  // a strided order (ascending page i goes to place i * stride mod n_order, a
+  // bijection for stride coprime to n_order): neighbouring pages tend to be
   // selected by the same rows, and spreading them out evens the work of the
   // waves over any window of pages.  Where they share few, ascending order:
   // the tiles running side by side on an XCD then reach a shared page at
   // nearly the same time, while it is still in that XCD's L2, and the waves'
   // work is even anyway.  The stride is the first odd number from 7 on that is
-  // coprime to n_union: 7, else 9, 11, 13 (15 shares the 3 that ruled 9 out),
-  // else 17 (a union that 3, 7, 11 and 13 divide is 3003 pages).
-  static_assert(MAX_UNION < 2 * 3003, "17 is coprime to a union that rules out the others");
+  // coprime to n_order: 7, else 9, 11, 13 (15 shares the 3 that ruled 9 out),
+  // else 17 (a length that 3, 7, 11 and 13 divide is 3003 pages).
+  static_assert(MAX_ORDER < 2 * 3003, "17 is coprime to a length that rules out the others");
   int stride = 1;
-  if (n_union > 1 && 10 * n_rows * take >= LS_ATT_SHARE_STRIDED * n_union)
-    stride = n_union % 7 ? 7 : n_union % 3 ? 9 : n_union % 11 ? 11 : n_union % 13 ? 13 : 17;
+  if (n_order > 1 && 10 * n_grp * take >= LS_ATT_SHARE_STRIDED * n_order)
+    stride = n_order % 7 ? 7 : n_order % 3 ? 9 : n_order % 11 ? 11 : n_order % 13 ? 13 : 17;
   for (int sg = seg0; sg < seg1; ++sg) {
     const int page = 64 * sg + lane;
     const uint32_t rows = page <= last_page ? s_rows[page] : 0u;
@@ -400,26 +433,36 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
     const int pos = (int)__builtin_amdgcn_mbcnt_hi(
         (uint32_t)(mk >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mk, (uint32_t)pos0));
     if (rows != 0u) {
-      const int dst = (int)(((uint32_t)pos * (uint32_t)stride) % (uint32_t)n_union);
-      int n_waves = 0;
-#pragma unroll
-      for (int i = 0; i < LS_ATT_WAVES; ++i) n_waves += ((rows >> (TPW * i)) & ROWS_MASK) != 0u;
-      s_umeta[dst] = rows;
-      s_upage[dst] = (uint16_t)page;
-      s_uneed[dst] = (uint8_t)n_waves;
+      const int dst = (int)(((uint32_t)pos * (uint32_t)stride) % (uint32_t)n_order);
+      s_omask[dst] = rows;
+      s_opage[dst] = (uint16_t)page;
     }
     pos0 += __popcll(mk);
   }
   __syncthreads();
-  // This wave's pages, in union order.
-  int n_visits = 0;
-  for (int u0 = 0; u0 < n_union; u0 += 64) {
+  // The tile's pages of the order are its union; every wave finds their places
+  // there (the waves take turns to write them down) and its own pages among them.
+  int n_union = 0, n_visits = 0;
+  for (int u0 = 0; u0 < n_order; u0 += 64) {
     const int u = u0 + lane;
-    const uint32_t rows = u < n_union ? (s_umeta[u] >> (TPW * w)) & ROWS_MASK : 0u;
-    const uint64_t mk = __ballot(rows != 0u);
+    const uint32_t rows = u < n_order ? (s_omask[u] >> off) & TILE_MASK : 0u;
+    const uint32_t mine = (rows >> w0) & rows_mask;
+    const uint64_t tk = __ballot(rows != 0u), mk = __ballot(mine != 0u);
+    const int ui = (int)__builtin_amdgcn_mbcnt_hi(
+        (uint32_t)(tk >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)tk, (uint32_t)n_union));
     const int pos = (int)__builtin_amdgcn_mbcnt_hi(
         (uint32_t)(mk >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mk, (uint32_t)n_visits));
-    if (rows != 0u) s_wlist[w][pos] = (uint32_t)s_upage[u] | rows << 13 | (uint32_t)u << 16;
+    const int page = u < n_order ? (int)s_opage[u] : 0;
+    if (mine != 0u) s_wlist[w][pos] = (uint32_t)page | mine << 13 | (uint32_t)ui << 16;
+    if ((u0 / 64) % LS_ATT_WAVES == w && rows != 0u) {
+      int n_waves = 0;
+#pragma unroll
+      for (int i = 0; i < LS_ATT_WAVES; ++i)
+        n_waves += ((rows >> LsAttTile<TPW>::row0(i)) & ((1u << LsAttTile<TPW>::rows(i)) - 1u)) != 0u;
+      s_upage[ui] = (uint16_t)page;
+      s_uneed[ui] = (uint8_t)n_waves;
+    }
+    n_union += __popcll(tk);
     n_visits += __popcll(mk);
   }
   __syncthreads();  // the lists are complete and the tables are dead, so the
@@ -658,7 +701,7 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
     e_cur = uniform(e_next);
     e_next = entry(k + 2);
     const int page = (int)(e & 0x1fffu);
-    const uint32_t sel = (e >> 13) & ROWS_MASK;
+    const uint32_t sel = (e >> 13) & ((1u << TPW) - 1u);
     const float p_unscale = uniform_f(__builtin_ldexpf(1.f, -v_e));
     const uint64_t ve_mask = v_e > 7 ? ~0ull : 0ull;
     load_k(ui, 0);
@@ -686,10 +729,10 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
                         LS_ATTN_RING_TIMEOUT) != 0;
 #pragma unroll
   for (int j = 0; j < TPW; ++j) {
-    const int row = w * TPW + j;
+    const int row = w0 + j;
     float l_tot = l_run[j] + ls_shfl_xor(l_run[j], 16);
     l_tot += ls_shfl_xor(l_tot, 32);
-    if (row >= n_rows || !head_ok) continue;
+    if (j >= n_mine || row >= n_rows || !head_ok) continue;
     const int64_t t = t0 + row;
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     uint16_t* orow = out + (t * G * gs + (int64_t)g * gs + head) * D + 4 * q;
@@ -766,22 +809,27 @@ struct AttnTiling {
   int tpw, run, span, per_xcd;
 };
 
-// One workgroup fills a CU's LDS, so a call runs in rounds of 256 tiles.  Three
-// rows a wave (24-row tiles) share each page copy among the most rows, but a call
-// of few rows then leaves CUs idle, or a second round nearly empty: while the
-// smaller tile still gives at most two rounds it is the faster one (attention of
-// one sequence, us, tiles of 8 / 16 / 24 rows: 600 rows 28 / 36 / 44, 2000 70 / 79
-// / 98, 2300 91 / 88 / 107, 4096 194 / 156 / 178, 4700 255 / 210 / 200).  Runs of 4
-// tiles even the XCDs' loads where runs of 16 leave some idle (8K rows 411 against
-// 463 us, 4096 rows 174 against 210) and cost nothing at 128K (12.06 against
-// 12.08 ms).  An XCD that alternates between the KV groups run by run starts every
-// group's large tiles early, which a call of up to four rounds needs (three
-// sequences of 4500 rows 106 against 134 us); longer calls keep to one group at a
-// time, whose pages then have the XCD's L2 to themselves (128K 12.06 against 12.42
-// ms, four sequences of 24K rows 1.20 against 1.25).
+int attn_tile_rows(int tpw) {
+  return tpw == 1 ? LsAttTile<1>::kTile : tpw == 2 ? LsAttTile<2>::kTile : LsAttTile<3>::kTile;
+}
+
+// One workgroup fills a CU's LDS, so a call runs in rounds of 256 tiles.  24-row
+// tiles share each page copy among the most rows, but a call of few rows then
+// leaves CUs idle and waits for its largest tile: while a smaller tile gives at
+// most two rounds it is the faster one (the attention call of one sequence, us,
+// tiles of 8 / 12 / 24 rows: 600 rows 43 / 47 / 53, 2048 83 / 88 / 113, 2300 102 /
+// 95 / 122, 3072 146 / 129 / 153, 3400 174 / 164 / 172, 4096 217 / 217 / 205).
+// Runs of 4 tiles even the XCDs'
+// loads where runs of 16 leave some idle (8K rows 411 against 463 us) and cost
+// nothing at 128K (12.06 against 12.08 ms).  An XCD that
+// alternates between the KV groups run by run starts every group's large tiles
+// early, which a call of up to four rounds needs (three sequences of 4500 rows in
+// all 106 against 134 us); longer calls keep to one group at a time, whose pages
+// then have the XCD's L2 to themselves (128K 12.06 against 12.42 ms, four sequences
+// of 24K rows in all 1.20 against 1.25).
 AttnTiling attn_tiling(int64_t total_q, int batch, int G, int head_tiles) {
   constexpr int64_t kCus = 256;
-  auto tiles = [&](int tpw) { return (total_q + LS_ATT_WAVES * tpw - 1) / (LS_ATT_WAVES * tpw); };
+  auto tiles = [&](int tpw) { return (total_q + attn_tile_rows(tpw) - 1) / attn_tile_rows(tpw); };
   const int64_t per_tile = (int64_t)G * head_tiles;
   AttnTiling t;
   t.tpw = tiles(1) * per_tile <= 2 * kCus ? 1 : tiles(2) * per_tile <= 2 * kCus ? 2 : 3;
@@ -854,7 +902,7 @@ int attn_run(const char* who, const void* q, int64_t q_row_stride, const void* k
   int32_t* status = status_out ? status_out : (int32_t*)(ws + L.status);
   const int gs = num_heads / num_kv_heads;
   const AttnTiling tl = attn_tiling(total_q, batch, num_kv_heads, (gs + 15) / 16);
-  const int tile_rows = LS_ATT_WAVES * tl.tpw;
+  const int tile_rows = attn_tile_rows(tl.tpw);
   hipLaunchKernelGGL(ls_attn_plan_kernel, dim3(1), dim3(64), 0, s, cu_seqlens_q, cu_seqlens_k,
                      batch, tile_rows, pg, tiles, tok, LS_ATT_UNION_CAP + 1, status);
   int rc = ls_check_launch("ls_attn_plan_kernel");

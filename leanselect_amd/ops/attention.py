@@ -16,7 +16,7 @@ def attention_tile_rows(take: int) -> int:
     """Most query rows per workgroup of the attention kernel for plans of ``take`` ids a
     row: 24 (three rows per wave) for every width it accepts (at most 128 ids; the
     union of a tile is at most 3072 pages).  Calls of few rows are cut into tiles of 8
-    or 16 rows (``attn_tiling`` in csrc/ls_attention.hip)."""
+    or 12 rows (``attn_tiling`` in csrc/ls_attention.hip)."""
     if take > 128:
         raise ValueError("the attention kernel accepts at most 128 ids per row")
     return 24

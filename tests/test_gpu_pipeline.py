@@ -238,11 +238,11 @@ def test_attention_every_row_of_a_ragged_batch():
 
 
 @pytest.mark.parametrize("lens", [(1,), (9, 1, 40), (2048,), (2049,), (4095, 1), (4097,),
-                                  (12288,), (12289,), (2000, 1000, 1500)])
+                                  (12288,), (12289,), (2000, 1000, 1500), (3072,), (3073,)])
 @pytest.mark.parametrize("biased", [False, True])
 def test_attention_tile_sizes_and_tile_deal(lens, biased):
-    """Calls on both sides of the launcher's lines between 8-, 16- and 24-row tiles
-    (two KV groups: 2048 and 4096 rows) and between the two orders of the tile deal
+    """Calls on both sides of the launcher's lines between 8-, 12- and 24-row tiles
+    (two KV groups: 2048 and 3072 rows) and between the two orders of the tile deal
     (12288 rows): every row is written, and sampled rows match the oracle, with and
     without the NOSA key bias."""
     case, ids = _attention_case(lens=lens, seed=14)
@@ -289,6 +289,41 @@ def test_attention_lse_of_one_key_is_its_score(n, amp):
     assert bool(((got - want).abs() <= 2.5 * 2.0 ** -24 * want.abs()).all())
     assert torch.equal(out.cpu()[rows].float().view(-1, G, H // G, D),
                        v[rows].float()[:, :, None].expand(-1, G, H // G, D))
+
+
+@pytest.mark.parametrize("biased", [False, True])
+def test_attention_is_independent_of_packing(biased):
+    """A sequence gives the same bits alone, in a small call and in a large one,
+    whichever tile height each of those calls takes: short sequences, one of a
+    whole number of 24-row groups, one row more and one row less among them, with
+    plans that share many pages (strided order) and few (ascending order)."""
+    lens = (1337, 48, 71, 1, 649, 2900)
+    case, ids = _attention_case(lens=lens, seed=17)
+    G, N, T = ids.shape
+    gen = torch.Generator().manual_seed(18)
+    cu = case.cu_host
+    for t in range(cu[5] + 1500, N):  # few shared pages: single random ids
+        n = (t - cu[5]) // 64 + 1
+        ids[:, t] = -1
+        ids[:, t, :3] = torch.randint(0, n, (G, 3), generator=gen, dtype=torch.int32).to(DEV)
+    cis = torch.randn(N, G, generator=gen).to(case.q.dtype).to(DEV)
+
+    def attend(first, last):
+        s, e = cu[first], cu[last]
+        off = torch.tensor([x - s for x in cu[first:last + 1]], dtype=torch.int32, device=DEV)
+        longest = max(lens[first:last])
+        qkv = (case.q[s:e], case.k[s:e], case.v[s:e])
+        plan = ids[:, s:e].contiguous()
+        if biased:
+            return nosa_sparse_attention(*qkv, cis[s:e], off, off, longest, longest, plan), None
+        return sparse_attention(*qkv, off, off, longest, longest, plan, return_lse=True)
+
+    out, lse = attend(0, len(lens))
+    for first, last in [(b, b + 1) for b in range(len(lens))] + [(0, 2), (1, 5), (0, 5)]:
+        one, one_lse = attend(first, last)
+        assert torch.equal(one, out[cu[first]:cu[last]])
+        if lse is not None:
+            assert torch.equal(one_lse, lse[:, cu[first]:cu[last]])
 
 
 def test_attention_messy_ids_duplicates_unsorted_out_of_range():
