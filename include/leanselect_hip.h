@@ -293,6 +293,16 @@ int ls_sparse_attn_varlen_noalloc(const void* q, int64_t q_row_stride, const voi
  */
 int32_t ls_attn_set_spin_limit(int32_t spins);
 
+/*
+ * Query rows per workgroup that the prefill attention entry points take for a
+ * call of these sizes: 8, 12 or 24 (0 for sizes they don't accept).  It only
+ * tells how the work is cut: a sequence's outputs are bit for bit the same at
+ * every height, whatever else is packed into the call.  Touches no device.  No
+ * counterpart in the reference.
+ */
+int32_t ls_attn_tile_rows(int64_t total_q, int32_t batch, int32_t num_heads,
+                          int32_t num_kv_heads, int32_t max_seqlen_k);
+
 /* ------------------------------------------------------------------------ */
 /* NOSA variant (leanselect/models/nosa.py, --method leanselect)             */
 /* ------------------------------------------------------------------------ */

@@ -819,23 +819,30 @@ int attn_tile_rows(int tpw) {
 // most two rounds it is the faster one (the attention call of one sequence, us,
 // tiles of 8 / 12 / 24 rows: 600 rows 43 / 47 / 53, 2048 83 / 88 / 113, 2300 102 /
 // 95 / 122, 3072 146 / 129 / 153, 3400 174 / 164 / 172, 4096 217 / 217 / 205).
-// Runs of 4 tiles even the XCDs'
+// Sequences of up to 256 keys have few pages, so a round takes about as long at
+// every height (it is mostly the tile's setup) and one round of larger tiles beats
+// two of smaller ones (100 sequences of 20 rows 56 / 55 / 50, 40 of 64 rows 55 / 54
+// / 44, 20 of 40 rows, one round, 35 / 36 / 41).  Runs of 4 tiles even the XCDs'
 // loads where runs of 16 leave some idle (8K rows 411 against 463 us) and cost
-// nothing at 128K (12.06 against 12.08 ms).  An XCD that
-// alternates between the KV groups run by run starts every group's large tiles
-// early, which a call of up to four rounds needs (three sequences of 4500 rows in
-// all 106 against 134 us); longer calls keep to one group at a time, whose pages
-// then have the XCD's L2 to themselves (128K 12.06 against 12.42 ms, four sequences
-// of 24K rows in all 1.20 against 1.25).
-AttnTiling attn_tiling(int64_t total_q, int batch, int G, int head_tiles) {
+// nothing at 128K (12.06 against 12.08 ms).  An XCD that alternates between the KV
+// groups run by run starts every group's large tiles early, which a call of up to
+// four rounds needs (three sequences of 4500 rows in all 106 against 134 us);
+// longer calls keep to one group at a time, whose pages then have the XCD's L2 to
+// themselves (128K 12.06 against 12.42 ms, four sequences of 24K rows in all 1.20
+// against 1.25).
+AttnTiling attn_tiling(int64_t total_q, int batch, int G, int head_tiles, int max_seqlen_k) {
   constexpr int64_t kCus = 256;
-  auto tiles = [&](int tpw) { return (total_q + attn_tile_rows(tpw) - 1) / attn_tile_rows(tpw); };
+  // At most this many tiles of one group: each sequence's last tile may be partial.
+  auto tiles = [&](int tpw) {
+    const int rows = attn_tile_rows(tpw);
+    return (total_q + (int64_t)batch * (rows - 1)) / rows;
+  };
   const int64_t per_tile = (int64_t)G * head_tiles;
+  const int64_t most = (max_seqlen_k <= 256 ? 1 : 2) * kCus;
   AttnTiling t;
-  t.tpw = tiles(1) * per_tile <= 2 * kCus ? 1 : tiles(2) * per_tile <= 2 * kCus ? 2 : 3;
+  t.tpw = tiles(1) * per_tile <= most ? 1 : tiles(2) * per_tile <= most ? 2 : 3;
   t.run = 4;
-  const int64_t bound = tiles(t.tpw) + batch;  // each sequence's last tile may be partial
-  t.per_xcd = (int)(t.run * ((bound + 8 * t.run - 1) / (8 * t.run)));
+  t.per_xcd = (int)(t.run * ((tiles(t.tpw) + 8 * t.run - 1) / (8 * t.run)));
   t.span = tiles(t.tpw) * per_tile <= 4 * kCus ? t.run : t.per_xcd;
   return t;
 }
@@ -901,7 +908,8 @@ int attn_run(const char* who, const void* q, int64_t q_row_stride, const void* k
   int32_t* tok = (int32_t*)(ws + L.tok);
   int32_t* status = status_out ? status_out : (int32_t*)(ws + L.status);
   const int gs = num_heads / num_kv_heads;
-  const AttnTiling tl = attn_tiling(total_q, batch, num_kv_heads, (gs + 15) / 16);
+  const AttnTiling tl =
+      attn_tiling(total_q, batch, num_kv_heads, (gs + 15) / 16, max_seqlen_k);
   const int tile_rows = attn_tile_rows(tl.tpw);
   hipLaunchKernelGGL(ls_attn_plan_kernel, dim3(1), dim3(64), 0, s, cu_seqlens_q, cu_seqlens_k,
                      batch, tile_rows, pg, tiles, tok, LS_ATT_UNION_CAP + 1, status);
@@ -961,6 +969,15 @@ extern "C" int32_t ls_attn_set_spin_limit(int32_t spins) {
   const int32_t prev = g_spin_limit;
   g_spin_limit = spins < 0 ? kDefaultSpinLimit : spins;
   return prev;
+}
+
+extern "C" int32_t ls_attn_tile_rows(int64_t total_q, int32_t batch, int32_t num_heads,
+                                     int32_t num_kv_heads, int32_t max_seqlen_k) {
+  if (total_q < 0 || batch < 0 || num_kv_heads <= 0 || num_heads <= 0 ||
+      num_heads % num_kv_heads != 0)
+    return 0;
+  const int head_tiles = (num_heads / num_kv_heads + 15) / 16;
+  return attn_tile_rows(attn_tiling(total_q, batch, num_kv_heads, head_tiles, max_seqlen_k).tpw);
 }
 
 extern "C" size_t ls_sparse_attn_workspace_size(int64_t total_k, int32_t batch,

@@ -15,8 +15,9 @@ __all__ = ["attention_tile_rows", "infllmv2_attn_varlen_func", "sparse_attention
 def attention_tile_rows(take: int) -> int:
     """Most query rows per workgroup of the attention kernel for plans of ``take`` ids a
     row: 24 (three rows per wave) for every width it accepts (at most 128 ids; the
-    union of a tile is at most 3072 pages).  Calls of few rows are cut into tiles of 8
-    or 12 rows (``attn_tiling`` in csrc/ls_attention.hip)."""
+    union of a tile is at most 3072 pages).  The visit order of a row's pages comes
+    from 24 rows in every call; ``_hip.lib().ls_attn_tile_rows`` gives the rows per
+    workgroup of one call (8 or 12 where it has few rows)."""
     if take > 128:
         raise ValueError("the attention kernel accepts at most 128 ids per row")
     return 24

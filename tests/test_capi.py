@@ -53,6 +53,24 @@ def test_invalid_arguments_fail_before_any_launch():
     assert rc == _hip.LS_ERR_INVALID and b"take" in lib.ls_last_error()
 
 
+@pytest.mark.parametrize("lens,rows", [
+    ((2048,), 8), ((2049,), 12), ((3072,), 12), ((3073,), 24), ((131072,), 24), ((1000, 1000), 8),
+    # Partial tiles count: 100 x 40 rows are 600 tiles of 8 rows in each of two groups.
+    ((20,) * 100, 24), ((40,) * 100, 24), ((64,) * 40, 24), ((40,) * 20, 8), ((1,), 8), ((), 8),
+    ((1025, 1025), 12), ((300,) * 6, 8)])
+def test_attention_tile_rows_follow_the_calls_tiles(lens, rows):
+    """At most two rounds of 256 workgroups (one for sequences of up to 256 keys)
+    for tiles of 8 or 12 rows, each sequence's last tile counted whole."""
+    lib = _hip.lib()
+    assert lib.ls_attn_tile_rows(sum(lens), len(lens), 32, 2, max(lens, default=0)) == rows
+    if rows < 24:
+        tiles = 2 * sum(-(-n // rows) for n in lens)
+        assert tiles <= (256 if max(lens, default=0) <= 256 else 512)
+    # Four times the tiles (KV groups or heads per group) reach the next height sooner.
+    assert lib.ls_attn_tile_rows(sum(lens), len(lens), 128, 8, max(lens, default=0)) >= rows
+    assert lib.ls_attn_tile_rows(sum(lens), len(lens), 32, 3, 0) == 0  # heads not divisible
+
+
 def test_nosa_entry_points_validate_before_any_launch():
     lib = _hip.lib()
     B = _hip.LS_BF16

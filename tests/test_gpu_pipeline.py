@@ -238,11 +238,13 @@ def test_attention_every_row_of_a_ragged_batch():
 
 
 @pytest.mark.parametrize("lens", [(1,), (9, 1, 40), (2048,), (2049,), (4095, 1), (4097,),
-                                  (12288,), (12289,), (2000, 1000, 1500), (3072,), (3073,)])
+                                  (12288,), (12289,), (2000, 1000, 1500), (3072,), (3073,),
+                                  (20,) * 100, (40,) * 24])
 @pytest.mark.parametrize("biased", [False, True])
 def test_attention_tile_sizes_and_tile_deal(lens, biased):
     """Calls on both sides of the launcher's lines between 8-, 12- and 24-row tiles
-    (two KV groups: 2048 and 3072 rows) and between the two orders of the tile deal
+    (two KV groups: 2048 and 3072 rows, or 1024 and 1536 in short sequences, each
+    counted with its partial tiles) and between the two orders of the tile deal
     (12288 rows): every row is written, and sampled rows match the oracle, with and
     without the NOSA key bias."""
     case, ids = _attention_case(lens=lens, seed=14)
