@@ -293,17 +293,21 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
   const int w0 = LsAttTile<TPW>::row0(w), n_mine = LsAttTile<TPW>::rows(w);
   const uint32_t rows_mask = (1u << n_mine) - 1u;
 
-  // XCD-aware tile order.  Consecutive workgroups land on different XCDs
-  // (workgroup x runs on XCD x % 8).  Each XCD takes runs of `run` consecutive
+  // XCD-aware tile order.  The grid is 8 * per_xcd workgroups by the KV groups,
+  // numbered as they are started, x first; consecutive workgroups land on different
+  // XCDs (workgroup i runs on XCD i % 8).  Each XCD takes runs of `run` consecutive
   // tiles, so the tiles in flight on one XCD are neighbours that share pages in
   // its L2, and turns to the next KV group every `span` tiles (a multiple of
   // run).  The runs are dealt over the XCDs there and back (0..7, then 7..0), and
   // from the end of the sequence first, so every XCD gets an even share of late
   // (large-union) and early (small-union) rows, the largest tiles start first and
-  // small ones fill the tail.  The grid is 8 * G * (a multiple of span), so this
-  // is a permutation of the workgroup indices.
-  const int xcd = LS_BID_X % 8, xi = LS_BID_X / 8;
-  const int turn = xi / span, g = turn % G, at = turn / G * span + xi % span;
+  // small ones fill the tail.  per_xcd is a multiple of span, so this is a
+  // permutation of the workgroups.
+  const int xcd = LS_BID_X % 8;
+  const uint32_t xi = (uint32_t)LS_BID_Y * (uint32_t)per_xcd + (uint32_t)(LS_BID_X / 8);
+  const uint32_t turn = xi / (uint32_t)span;
+  const int g = (int)(turn % (uint32_t)G);
+  const int at = (int)(turn / (uint32_t)G * (uint32_t)span + xi % (uint32_t)span);
   const int deal = at / run;
   const int64_t tile = 8LL * per_xcd - 1 -
                        ((int64_t)(8 * deal + ((deal & 1) ? 7 - xcd : xcd)) * run + at % run);
@@ -941,7 +945,7 @@ int attn_run(const char* who, const void* q, int64_t q_row_stride, const void* k
   }
   const float scale = softmax_scale > 0.f ? softmax_scale : 1.0f / sqrtf((float)head_dim);
   const float scale_log2 = scale * 1.4426950408889634f;
-  const dim3 grid((unsigned)(8 * tl.per_xcd * num_kv_heads), 1, (gs + 15) / 16);
+  const dim3 grid((unsigned)(8 * tl.per_xcd), num_kv_heads, (gs + 15) / 16);
 #define LS_TILE_ARGS                                                                              \
   grid, s, q, q_row_stride, kv, L, vexp, cb, tok, cu_seqlens_q, cu_seqlens_k, pg,              \
       tiles, batch, total_q, num_kv_heads, gs, topk_idx, take, scale_log2, causal, out, lse, \

@@ -328,6 +328,33 @@ def test_attention_is_independent_of_packing(biased):
             assert torch.equal(one_lse, lse[:, cu[first]:cu[last]])
 
 
+def test_attention_grid_holds_many_rows_times_groups():
+    """Tiles x KV groups x 512 threads = 2^32, past what one grid dimension holds:
+    plans without pages and one query row read for all (row stride 0), so that only
+    the 52 GB output has the call's size.  Rows of every part of the grid are written."""
+    G, D, n = 32, 128, 24 * (1 << 18)
+    if torch.cuda.mem_get_info()[0] < 60 << 30:
+        pytest.skip("needs 52 GB for the output")
+    q = torch.ones(1, G, D, dtype=torch.bfloat16, device=DEV)
+    k = torch.ones(64, G, D, dtype=torch.bfloat16, device=DEV)
+    out = torch.empty(n, G, D, dtype=torch.bfloat16, device=DEV)
+    rows = torch.arange(0, n, 4999, device=DEV)
+    out[rows] = float("nan")
+    out[-1] = float("nan")
+    cu_q = torch.tensor([0, n], dtype=torch.int32, device=DEV)
+    cu_k = torch.tensor([0, 64], dtype=torch.int32, device=DEV)
+    L = _hip.lib()
+    assert L.ls_attn_tile_rows(n, 1, G, G, 64) * (1 << 18) == n
+    ws = _hip.workspace(L.ls_sparse_attn_workspace_size(64, 1, G, D, 64, _hip.LS_BF16), k.device)
+    rc = L.ls_sparse_attn_varlen(
+        q.data_ptr(), 0, k.data_ptr(), G * D, k.data_ptr(), G * D, cu_q.data_ptr(),
+        cu_k.data_ptr(), 1, n, 64, n, 64, G, G, D, _hip.LS_BF16, None, 0, 64, -1.0, 0,
+        out.data_ptr(), None, ws.data_ptr(), ws.numel(), _hip.stream_of(k.device))
+    _hip.check(rc, "ls_sparse_attn_varlen")
+    torch.cuda.synchronize()
+    assert bool((out[rows] == 0).all()) and bool((out[-1] == 0).all())
+
+
 def test_attention_messy_ids_duplicates_unsorted_out_of_range():
     case, ids = _attention_case(lens=(1500,), seed=7)
     g = torch.Generator(device="cpu").manual_seed(0)
