@@ -270,8 +270,10 @@ def poll_attn_status() -> None:
 
 
 def stream_of(device: torch.device) -> int:
-    # The raw handle, without building a Stream object on every launch.
-    return torch._C._cuda_getCurrentRawStream(device.index)
+    # The raw handle, without building a Stream object on every launch.  A device
+    # without an index is the current one.
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def workspace(nbytes: int, device: torch.device) -> torch.Tensor:

@@ -6,7 +6,7 @@ import types
 import pytest
 import torch
 
-from leanselect_amd import minicpm
+from leanselect_amd import _hip, minicpm
 from leanselect_amd.ops import nosa_sparse_attention, sparse_attention
 
 
@@ -72,3 +72,10 @@ def test_prefill_rejects_empty_sequences(cu_host):
     ids = torch.zeros(10, dtype=torch.int32)
     with pytest.raises(ValueError, match="at least one token"):
         minicpm.MiniCPMLeanSelect.prefill(fake, ids, cu_host)
+
+
+def test_stream_of_a_device_without_an_index_is_the_current_devices(monkeypatch):
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 100 * index)
+    assert _hip.stream_of(torch.device("cuda")) == 300
+    assert _hip.stream_of(torch.device("cuda", 1)) == 100
