@@ -36,25 +36,30 @@ __host__ __device__ __forceinline__ int64_t ls_n_windows(int64_t len, int ks, in
 // Append, one launch.  The first n_append workgroups copy the packed new rows:
 // thread (row, g, chunk of 8 channels) copies 16 bytes of K and of V to position
 // cache_seqlens[b] + (row - cu_new[b]).  The others form the compressed windows
-// the new tokens complete: win_blocks workgroups per sequence, a pair of threads
-// per (window, g, 8 channels), each summing one half of the window's rows
+// the new tokens complete, the first max_windows of them in the order of the
+// sequences: a pair of threads per (window, g, 8 channels), each summing one half of the window's rows
 // [w*stride, w*stride + ks) in float32 in token order (windows of two strides;
 // other geometries are summed by the first thread alone).  The halves are
 // added, the order of the prefill's half-window kernel, so a window formed here
 // is bit-identical to the one the prefill forms from the same keys.  Rows of
 // this call are read from the new keys rather than the cache, so the windows
-// need not wait for the copies, and each workgroup finds its sequence's windows
-// from its lengths, without a prefix sum over the batch: what were three launches
-// in a chain (copy 1.8, plan 1.4, windows 5.3 us for one sequence; 3.3, 4.4, 9.5
-// for sixteen) are one.
+// need not wait for the copies, and each workgroup sums up the batch's new windows
+// itself (256 sequences at a time, in LDS), so they are dealt evenly over
+// the workgroups wherever in the batch they are: what were three launches in a
+// chain are one.  The call, three launches -> one, us: one sequence and one token
+// 18.6 -> 7.0, sixteen 24.1 -> 8.1, 64 sequences of which one gets 64K tokens
+// 62.7 -> 45.
 // ---------------------------------------------------------------------------
 template <int DT>
 __global__ __launch_bounds__(256) void ls_cache_append_kernel(
     uint16_t* kc_, uint16_t* __restrict__ vc_, int64_t cbs, int64_t crs,
     const int32_t* __restrict__ cache_seqlens, const uint16_t* __restrict__ kn,
     const uint16_t* __restrict__ vn, int64_t nrs, const int32_t* __restrict__ cu_new,
-    int64_t total_new, int batch, int G, int D, int64_t n_append, int win_blocks, int ks,
-    int stride, uint16_t* __restrict__ kcc, int64_t kbs, int64_t krs) {
+    int64_t total_new, int batch, int G, int D, int64_t n_append, int win_blocks,
+    int64_t max_windows, int ks, int stride, uint16_t* __restrict__ kcc, int64_t kbs,
+    int64_t krs) {
+  // Of each sequence of a pass: the new windows before it, its length, its first new row.
+  __shared__ int32_t s_off[256], s_len[256], s_new[256], s_sum[4];
   const int c8 = D / 8;
   const int64_t per_row = (int64_t)G * c8;
   const int64_t blk = blockIdx.x;
@@ -72,47 +77,79 @@ __global__ __launch_bounds__(256) void ls_cache_append_kernel(
     *reinterpret_cast<ls_u32x4*>(vc_ + dst) = ls_load16(vn + src);
     return;
   }
-  const int b = (int)((blk - n_append) / win_blocks);
-  const int64_t first = (blk - n_append) % win_blocks;
-  const int64_t l0 = cache_seqlens[b], n0 = cu_new[b];
-  const int64_t w0 = ls_n_windows(l0, ks, stride);
-  const int64_t n_win = ls_n_windows(l0 + (cu_new[b + 1] - n0), ks, stride) - w0;
   const int half = threadIdx.x & 1;
   const bool halves = ks == 2 * stride;
-  // Whole pairs leave the loop together (128 pairs per workgroup).
-  for (int64_t i = first * 128 + (threadIdx.x >> 1); i < n_win * per_row; i += 128LL * win_blocks) {
-    const int64_t wi = i / per_row;
-    const int rem = (int)(i - wi * per_row);
-    const int g = rem / c8, c = rem - g * c8;
-    const int64_t w = w0 + wi, p0 = w * stride;
-    const int64_t col = (int64_t)g * D + 8 * c;
-    const uint16_t* old_rows = kc_ + (int64_t)b * cbs + col;
-    const uint16_t* new_rows = kn + n0 * nrs + col;
-    const int r0 = halves ? half * stride : 0;
-    const int r1 = halves ? r0 + stride : (half ? 0 : ks);
-    float s[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) s[e] = 0.f;
-    // Unrolled so that a block of row loads is in flight at once; the sums
-    // still run in token order.
-#pragma unroll 16
-    for (int t = r0; t < r1; ++t) {
-      const int64_t p = p0 + t;
-      const ls_u32x4 a = ls_load16(p < l0 ? old_rows + p * crs : new_rows + (p - l0) * nrs);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        s[2 * e] += LsElem<DT>::to_f((uint16_t)(a[e] & 0xffffu));
-        s[2 * e + 1] += LsElem<DT>::to_f((uint16_t)(a[e] >> 16));
-      }
+  const int tid = threadIdx.x, lane = tid & 63;
+  auto windows = [&](int32_t len) {  // ls_n_windows in 32 bits
+    return len >= ks ? (int32_t)((uint32_t)(len - ks) / (uint32_t)stride) + 1 : 0;
+  };
+  for (int s0 = 0; s0 < batch && max_windows > 0; s0 += 256) {
+    int32_t mine = 0;
+    if (s0 + tid < batch) {
+      const int32_t len = cache_seqlens[s0 + tid], n0 = cu_new[s0 + tid];
+      mine = windows(len + (cu_new[s0 + tid + 1] - n0)) - windows(len);
+      s_len[tid] = len;
+      s_new[tid] = n0;
     }
-    const float n = (float)ks;
-    ls_u32x4 o;
+    int32_t before = mine;  // inclusive scan over the wave, then the workgroup
 #pragma unroll
-    for (int e = 0; e < 8; ++e) s[e] = (s[e] + ls_shfl_xor(s[e], 1)) / n;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int32_t y = __shfl_up(before, d, 64);
+      if (lane >= d) before += y;
+    }
+    if (lane == 63) s_sum[tid >> 6] = before;
+    before -= mine;
+    __syncthreads();
+    int64_t n_win = 0;
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-      o[e] = ls_pack2(LsElem<DT>::from_f(s[2 * e]), LsElem<DT>::from_f(s[2 * e + 1]));
-    if (!half) *reinterpret_cast<ls_u32x4*>(kcc + (int64_t)b * kbs + w * krs + col) = o;
+    for (int i = 0; i < 4; ++i) {
+      if (i < tid >> 6) before += s_sum[i];
+      n_win += s_sum[i];
+    }
+    s_off[tid] = before;
+    __syncthreads();
+    n_win = n_win < max_windows ? n_win : max_windows;
+    max_windows -= n_win;
+    const int n_seq = batch - s0 < 256 ? batch - s0 : 256;
+    // Whole pairs leave the loop together (128 pairs per workgroup).
+    for (int64_t i = (blk - n_append) * 128 + (tid >> 1); i < n_win * per_row;
+         i += 128LL * win_blocks) {
+      const int64_t wi = i / per_row;
+      const int rem = (int)(i - wi * per_row);
+      const int g = rem / c8, c = rem - g * c8;
+      const int bs = ls_find_segment(s_off, n_seq, wi), b = s0 + bs;
+      const int64_t l0 = s_len[bs], n0 = s_new[bs];
+      const int64_t w = windows((int32_t)l0) + (wi - s_off[bs]), p0 = w * stride;
+      const int64_t col = (int64_t)g * D + 8 * c;
+      const uint16_t* old_rows = kc_ + (int64_t)b * cbs + col;
+      const uint16_t* new_rows = kn + n0 * nrs + col;
+      const int r0 = halves ? half * stride : 0;
+      const int r1 = halves ? r0 + stride : (half ? 0 : ks);
+      float s[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s[e] = 0.f;
+      // Unrolled so that a block of row loads is in flight at once; the sums
+      // still run in token order.
+#pragma unroll 16
+      for (int t = r0; t < r1; ++t) {
+        const int64_t p = p0 + t;
+        const ls_u32x4 a = ls_load16(p < l0 ? old_rows + p * crs : new_rows + (p - l0) * nrs);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          s[2 * e] += LsElem<DT>::to_f((uint16_t)(a[e] & 0xffffu));
+          s[2 * e + 1] += LsElem<DT>::to_f((uint16_t)(a[e] >> 16));
+        }
+      }
+      const float n = (float)ks;
+      ls_u32x4 o;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s[e] = (s[e] + ls_shfl_xor(s[e], 1)) / n;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        o[e] = ls_pack2(LsElem<DT>::from_f(s[2 * e]), LsElem<DT>::from_f(s[2 * e + 1]));
+      if (!half) *reinterpret_cast<ls_u32x4*>(kcc + (int64_t)b * kbs + w * krs + col) = o;
+    }
+    if (s0 + 256 < batch) __syncthreads();  // the tables are read before the next pass writes them
   }
 }
 
@@ -929,20 +966,18 @@ extern "C" int ls_kvcache_append(void* k_cache, void* v_cache, int64_t cache_bat
     LS_REQUIRE(cu_windows, LS_ERR_INVALID, "ls_kvcache_append: null cu_windows");
     LS_REQUIRE(ls_aligned16(kc_cache) && kc_row_stride % 8 == 0 && kc_batch_stride % 8 == 0,
                LS_ERR_UNSUPPORTED, "ls_kvcache_append: compressed cache must be 16-byte aligned");
-    // Enough workgroups for the whole batch's windows in one sequence, as far as
-    // the launch stays small (a workgroup then loops over more of its windows).
+    // Two rounds of the chip's threads at most: a workgroup then loops over its share.
     if (max_new_windows > 0 && n_append > 0)
-      win_blocks = std::min<int64_t>((max_new_windows * per_row + 127) / 128,
-                                     std::max<int64_t>(1, 4096 / batch));
+      win_blocks = std::min<int64_t>((max_new_windows * per_row + 127) / 128, 4096);
   }
-  const int64_t blocks = n_append + win_blocks * batch;
+  const int64_t blocks = n_append + win_blocks;
   if (blocks == 0) return LS_OK;
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, s, (uint16_t*)k_cache,
                        (uint16_t*)v_cache, cache_batch_stride, cache_row_stride, cache_seqlens,
                        (const uint16_t*)k_new, (const uint16_t*)v_new, new_row_stride,
                        cu_seqlens_new, total_new, batch, num_kv_heads, head_dim, n_append,
-                       (int)std::max<int64_t>(1, win_blocks), kernel_size, kernel_stride,
+                       (int)win_blocks, max_new_windows, kernel_size, kernel_stride,
                        (uint16_t*)kc_cache, kc_batch_stride, kc_row_stride);
   };
   dtype == LS_BF16 ? launch(ls_cache_append_kernel<LS_BF16>) : launch(ls_cache_append_kernel<LS_F16>);

@@ -11,7 +11,7 @@ import pytest
 import torch
 
 import oracle
-from leanselect_amd import minicpm
+from leanselect_amd import _hip, minicpm
 from leanselect_amd.infllm_v2 import (infllmv2_attn_stage1, infllmv2_attn_with_kvcache,
                                       max_pooling_1d_varlen)
 from leanselect_amd.ops import compress_k, decode_topk_idx, kvcache_append, sparse_attention_kvcache
@@ -388,6 +388,61 @@ def test_append_window_geometries(ks, stride, lens, n_new):
             assert bool(((kc[b, w0:w1].double() - want).abs()
                          <= 0.51 * oracle.output_step(want, torch.bfloat16) + 1e-6).all())
     assert torch.equal(k, want_k)
+
+
+@pytest.mark.parametrize("bound", [0, 1, 3, 4, 100])
+def test_append_writes_at_most_max_new_windows(bound):
+    """max_new_windows bounds what a call writes: of the four windows that this one
+    completes (one, none, two, one in its sequences) the first `bound`, in the order
+    of the sequences."""
+    lens, n_new, cap = [31, 40, 0, 63], [1, 1, 48, 1], 128
+    B = len(lens)
+    g = torch.Generator().manual_seed(43)
+    rnd = lambda *shape: torch.randn(*shape, generator=g).to(torch.bfloat16).to(DEV)  # noqa: E731
+    k, v = rnd(B, cap, G, D), rnd(B, cap, G, D)
+    kn, vn = rnd(sum(n_new), G, D), rnd(sum(n_new), G, D)
+    kc = torch.full((B, 7, G, D), 7.0, dtype=torch.bfloat16, device=DEV)
+    lt, cu = _i32(lens), _i32(_cu(n_new))
+    rc = _hip.lib().ls_kvcache_append(
+        k.data_ptr(), v.data_ptr(), k.stride(0), k.stride(1), lt.data_ptr(), kn.data_ptr(),
+        vn.data_ptr(), kn.stride(0), cu.data_ptr(), sum(n_new), B, G, D, _hip.LS_BF16,
+        kc.data_ptr(), kc.stride(0), kc.stride(1), bound, 32, 16,
+        torch.empty(B + 1, dtype=torch.int32, device=DEV).data_ptr(), _hip.stream_of(k.device))
+    _hip.check(rc, "ls_kvcache_append")
+    written = (kc != 7).flatten(2).any(-1).cpu()
+    places = [(0, 0), (2, 0), (2, 1), (3, 2)]
+    want = torch.zeros(B, 7, dtype=torch.bool)
+    for b, w in places[:bound]:
+        want[b, w] = True
+        rows = k[b, 16 * w:16 * w + 32].double()
+        assert bool(((kc[b, w].double() - rows.mean(0)).abs()
+                     <= 0.51 * oracle.output_step(rows.mean(0), torch.bfloat16) + 1e-6).all())
+    assert torch.equal(written, want)
+
+
+@pytest.mark.parametrize("B,long_at", [(70, 69), (256, 255), (600, 300)])
+def test_append_windows_of_one_long_sequence_in_a_large_batch(B, long_at):
+    """The windows of a batch are dealt over the launch wherever they are: one
+    sequence with many, the others with one or none, in batches below, at and past
+    the sequences that a workgroup sums up at a time."""
+    cap = 1024
+    lens = [(31, 40, 15, 0)[b % 4] for b in range(B)]
+    n_new = [1] * B
+    lens[long_at], n_new[long_at] = 16, 1000
+    g = torch.Generator().manual_seed(44)
+    k = torch.randn(B, cap, 1, 8, generator=g).to(torch.bfloat16).to(DEV)
+    kn = torch.randn(sum(n_new), 1, 8, generator=g).to(torch.bfloat16).to(DEV)
+    kc = torch.full((B, 64, 1, 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    kvcache_append(k, k.clone(), _i32(lens), kn, kn.clone(), _i32(_cu(n_new)), kc_cache=kc)
+    mean = k.double().unfold(1, 32, 16).mean(-1)
+    at = torch.arange(64)[None]
+    win = lambda n: ((n - 32) // 16 + 1).clamp_min(0)  # noqa: E731
+    l0, l1 = torch.tensor(lens)[:, None], torch.tensor([a + b for a, b in zip(lens, n_new)])[:, None]
+    new = ((at >= win(l0)) & (at < win(l1))).to(DEV)
+    assert int(new.sum()) == sum(b % 4 == 0 for b in range(B) if b != long_at) + 62
+    want = torch.cat([mean, torch.zeros_like(mean[:, :1])], 1)[:, :64]
+    err = (kc.double() - want).abs() <= 0.51 * oracle.output_step(want, torch.bfloat16) + 1e-6
+    assert bool(err[new].all()) and bool((kc[~new] == 7).all())
 
 
 @pytest.mark.parametrize("lens", [[1, 2], [64, 65], [63, 4097], [16384, 16385]])
