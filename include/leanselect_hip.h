@@ -510,8 +510,8 @@ int ls_embed_scale(const int32_t* ids, int64_t n, const void* table, int64_t voc
  * max_new_windows bounds the new windows of the whole batch: the first
  * max_new_windows of them, in the order of the sequences, are written (sum over
  * b of ceil(n_new(b) / kernel_stride) + batch always suffices).  cu_windows is
- * int32 [batch + 1] device scratch (required, no longer written).  The caller
- * guarantees cache_seqlens[b] + n_new(b) <= capacity and the windows fit kc_capacity.
+ * not used (null is fine).  The caller guarantees cache_seqlens[b] + n_new(b) <=
+ * capacity and that the windows fit kc_capacity.
  * Replaces DynamicLayer.update plus InfLLMv2CacheLayer.update_no_compress_k /
  * update_compress_k (leanselect/models/minicpm.py:1237-1325, called at
  * 2776-2823 and 2888-2958).

@@ -941,6 +941,7 @@ extern "C" int ls_kvcache_append(void* k_cache, void* v_cache, int64_t cache_bat
                                  void* kc_cache, int64_t kc_batch_stride, int64_t kc_row_stride,
                                  int64_t max_new_windows, int32_t kernel_size,
                                  int32_t kernel_stride, int32_t* cu_windows, void* stream) {
+  (void)cu_windows;
   LS_REQUIRE(batch >= 0 && total_new >= 0 && num_kv_heads > 0 && head_dim > 0, LS_ERR_INVALID,
              "ls_kvcache_append: bad sizes");
   LS_REQUIRE(dtype == LS_BF16 || dtype == LS_F16, LS_ERR_UNSUPPORTED,
@@ -963,7 +964,6 @@ extern "C" int ls_kvcache_append(void* k_cache, void* v_cache, int64_t cache_bat
   if (kc_cache && batch > 0) {
     LS_REQUIRE(kernel_size > 0 && kernel_stride > 0, LS_ERR_INVALID,
                "ls_kvcache_append: kernel_size and kernel_stride must be positive");
-    LS_REQUIRE(cu_windows, LS_ERR_INVALID, "ls_kvcache_append: null cu_windows");
     LS_REQUIRE(ls_aligned16(kc_cache) && kc_row_stride % 8 == 0 && kc_batch_stride % 8 == 0,
                LS_ERR_UNSUPPORTED, "ls_kvcache_append: compressed cache must be 16-byte aligned");
     // Two rounds of the chip's threads at most: a workgroup then loops over its share.

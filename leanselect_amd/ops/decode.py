@@ -90,7 +90,6 @@ def kvcache_append(k_cache: torch.Tensor, v_cache: torch.Tensor, cache_seqlens: 
     if not (k_new.stride(2) == 1 and k_new.stride(1) == D and v_new.stride() == k_new.stride()
             and k_new.stride(0) % 8 == 0):
         k_new, v_new = k_new.contiguous(), v_new.contiguous()
-    cu_win = torch.empty(B + 1, dtype=torch.int32, device=dev) if kc_cache is not None else None
     rc = _hip.lib().ls_kvcache_append(
         k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0), k_cache.stride(1),
         cache_seqlens.contiguous().data_ptr(), k_new.data_ptr(), v_new.data_ptr(), k_new.stride(0),
@@ -98,7 +97,7 @@ def kvcache_append(k_cache: torch.Tensor, v_cache: torch.Tensor, cache_seqlens: 
         _hip.dtype_code(k_cache.dtype), _hip.ptr(kc_cache),
         kc_cache.stride(0) if kc_cache is not None else 0,
         kc_cache.stride(1) if kc_cache is not None else 0, new_windows, int(kernel_size),
-        int(kernel_stride), _hip.ptr(cu_win), _hip.stream_of(dev))
+        int(kernel_stride), None, _hip.stream_of(dev))
     _hip.check(rc, "ls_kvcache_append")
 
 

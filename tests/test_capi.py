@@ -270,6 +270,13 @@ def test_fused_query_and_decode_entry_points_validate_before_any_launch():
     rc = lib.ls_sparse_attn_kvcache(None, 4096, None, 1, None, None, 0, 256, None, 1, 32, 2,
                                     128, B, None, 64, 0.088, 0, 65, None, None, None, 0, None)
     assert rc == _hip.LS_ERR_INVALID and b"n_splits" in lib.ls_last_error()
+    # ls_kvcache_append: no new rows is nothing to do, with or without a cu_windows buffer.
+    lens, kc = (ctypes.c_int32 * 2)(), ctypes.create_string_buffer(64)
+    addr, kc_at = ctypes.addressof(lens), -(-ctypes.addressof(kc) // 16) * 16
+    for cu_windows in (addr, None):
+        rc = lib.ls_kvcache_append(None, None, 0, 256, addr, None, None, 256, addr, 0, 1, 2, 128, B,
+                                   kc_at, 0, 256, 0, 32, 16, cu_windows, None)
+        assert rc == _hip.LS_OK
     # ls_dense_attn_kvcache: too many splits, null tensors.
     rc = lib.ls_dense_attn_kvcache(None, 4096, None, 1, None, None, 0, 256, None, 1, 32, 2,
                                    128, B, 0.088, 0, 65, None, None, None, 0, None)
