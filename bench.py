@@ -42,10 +42,9 @@ import torch
 ROOT = Path(__file__).resolve().parent
 sys.path.insert(0, str(ROOT))
 
-from leanselect_amd import workloads  # noqa: E402
+from leanselect_amd import _hip, workloads  # noqa: E402
 from leanselect_amd.ops import (compress_k, leanselect_prefill_topk_idx,  # noqa: E402
                                 nosa_prefill_topk_idx, nosa_sparse_attention, sparse_attention)
-from leanselect_amd.ops.attention import attention_tile_rows  # noqa: E402
 
 WORKLOADS = {
     "minicpm41_8b_layer_128k": dict(seq_lens=(131072,)),
@@ -90,10 +89,12 @@ def attention_keys(ids: torch.Tensor, cu_host: list[int]) -> int:
 def plan_locality(ids: torch.Tensor, cu_host: list[int], tile: int | None = None) -> dict:
     """Mean distinct pages of a ``tile``-row query tile's plans (per KV group), and
     the mean number of the tile's rows that chose each of those pages: how much
-    K/V one staged page serves. ``tile`` defaults to the attention kernel's."""
+    K/V one staged page serves. ``tile`` defaults to what the attention call of 16
+    query heads a group takes for these sequences."""
     G, N, T = ids.shape
     if tile is None:
-        tile = attention_tile_rows(T)
+        longest = max((b - a for a, b in zip(cu_host, cu_host[1:])), default=0)
+        tile = _hip.lib().ls_attn_tile_rows(N, len(cu_host) - 1, 16 * G, G, longest)
     unions, chosen = 0.0, 0.0
     n_tiles = 0
     for b in range(len(cu_host) - 1):

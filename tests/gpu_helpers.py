@@ -4,6 +4,13 @@ from __future__ import annotations
 import torch
 
 import oracle
+from leanselect_amd import _hip
+
+
+def tile_rows(q: torch.Tensor, k: torch.Tensor, cu_host: list[int], max_len: int) -> int:
+    """Query rows per workgroup of the attention call on ``q`` and ``k``."""
+    return _hip.lib().ls_attn_tile_rows(q.shape[0], len(cu_host) - 1, q.shape[1], k.shape[1],
+                                        max_len)
 
 
 def plan_structure_errors(ids: torch.Tensor, cu_host: list[int], take: int, init: int, local: int,

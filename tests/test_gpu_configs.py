@@ -16,7 +16,7 @@ import pytest
 import torch
 
 import oracle
-from gpu_helpers import oracle_select_rows, plan_structure_errors, spread_rows
+from gpu_helpers import oracle_select_rows, plan_structure_errors, spread_rows, tile_rows
 from leanselect_amd import minicpm, workloads
 from leanselect_amd.ops import (compress_k, leanselect_prefill_topk_idx, nosa_prefill_topk_idx,
                                 nosa_sparse_attention, sparse_attention)
@@ -270,21 +270,34 @@ def test_nosa_layer_128k():
     assert ok, (mx, mr)
 
 
-def test_attention_large_v_page_exponents():
+@pytest.mark.parametrize("n,height", [(1500, 8), (2900, 12), (4096, 24)])
+def test_attention_large_v_page_exponents(n, height):
     """Pages whose V exceeds fp16's range (|V| ~ 1e5 and ~ 1e7): the staged V^T
     carries a per-page power-of-two exponent, and exponents above 7 force the
     rescale path.  With values this large an output element can be a small
     difference of huge terms, so each element's error is bounded relative to
     the magnitude it is summed from, sum_j p_j |v_j|: 2^-10 of it covers the
     11-bit (fp16) weights of the P.V product plus the output's rounding (a
-    bf16 P, as the reference's kernel uses, would need 2^-7)."""
-    case = workloads.hidden_space_layer((4096,), device=DEV, seed=25)
+    bf16 P, as the reference's kernel uses, would need 2^-7).  At the shorter lengths
+    single elements also show the weights below fp16's normal range: P times the
+    page's 2^e is rounded to 2^-25 there, which is 2^-25 2^-e |v_j| of the output per
+    key (the weights' sum is at least 1), and that sum over the row's pages is added
+    to the bound; there the bits must also be those of a call of 24-row tiles."""
+    case = workloads.hidden_space_layer((n,), device=DEV, seed=25)
+    assert tile_rows(case.q, case.k, case.cu_host, n) == height
     _, _, ids = _select(case)
     v = case.v.clone()
-    for p, scale in ((0, 1e5), (3, 1e7), (17, 3e4), (40, 2e6)):
+    for p, scale in ((0, 1e5), (3, 1e7), (17, 3e4), (min(40, n // 64 - 1), 2e6)):
         v[64 * p : 64 * p + 64] = (v[64 * p : 64 * p + 64].float() * scale).to(v.dtype)
     assert float(v.float().abs().max()) > 32768 * 128
-    out = sparse_attention(case.q, case.k, v, case.cu_seqlens, case.cu_seqlens, 4096, 4096, ids)
+    out = sparse_attention(case.q, case.k, v, case.cu_seqlens, case.cu_seqlens, n, n, ids)
+    if height != 24:
+        three = lambda x: torch.cat([x] * 3)  # noqa: E731
+        cu = torch.arange(0, 3 * n + 1, n, dtype=torch.int32, device=DEV)
+        q3, k3 = three(case.q), three(case.k)
+        assert tile_rows(q3, k3, [0, n, 2 * n, 3 * n], n) == 24
+        again = sparse_attention(q3, k3, three(v), cu, cu, n, n, torch.cat([ids] * 3, 1))
+        assert all(torch.equal(x, out) for x in again.split(n))
     rows = spread_rows(case.cu_host, per_seq=64)
     want, _, mass = oracle.sparse_attention(case.q.cpu(), case.k.cpu(), v.cpu(), case.cu_host,
                                             case.cu_host, ids.cpu()[:, rows], rows=rows,
@@ -293,6 +306,17 @@ def test_attention_large_v_page_exponents():
     b = want.double()
     err = (got - b).abs()
     bound = 2.0 ** -10 * mass + oracle.output_step(b, torch.bfloat16)
+    if n < 4096:
+        G, D = case.k.shape[1:]
+        va = torch.zeros(-(-n // 64) * 64, G, D, dtype=torch.float64)
+        va[:n] = v.cpu().double().abs()
+        va = va.view(-1, 64, G, D)
+        e = torch.ceil(torch.log2(va.amax((1, 3)) / 32768)).clamp(0, 15)
+        tail = 2.0 ** (-25 - e)[..., None] * va.sum(1)  # [pages, G, D]
+        plan = ids.cpu()[:, rows].long()
+        for g in range(G):
+            per_page = torch.where((plan[g] >= 0)[..., None], tail[plan[g].clamp_min(0), g], 0.0)
+            bound[:, g * 16:(g + 1) * 16] += per_page.sum(1)[:, None]
     worst = float((err / bound).max())
     mr = float(err.mean() / b.abs().mean())
     print(f"\nlarge-V attention: worst error / bound = {worst:.3f} mean_rel={mr:.3e}", flush=True)
@@ -300,10 +324,13 @@ def test_attention_large_v_page_exponents():
     assert bool(torch.isfinite(out).all())
 
 
-def test_attention_queries_shorter_than_keys():
+@pytest.mark.parametrize("lens_q,lens_k,height", [
+    ((100, 700, 1, 600), (300, 700, 65, 1700), 8),
+    ((100, 700, 1500, 1), (300, 700, 2600, 65), 12),
+    ((100, 700, 2600, 1), (300, 700, 3700, 65), 24)])
+def test_attention_queries_shorter_than_keys(lens_q, lens_k, height):
     """len_q < len_k per sequence under causal=True: row t of a sequence sees keys
     j <= t + len_k - len_q (the queries are the last len_q positions)."""
-    lens_q, lens_k = (100, 700, 1500, 1), (300, 700, 2600, 65)
     cq, ck = [0], [0]
     for a, b in zip(lens_q, lens_k):
         cq.append(cq[-1] + a)
@@ -322,6 +349,7 @@ def test_attention_queries_shorter_than_keys():
                 ids[gg, cq[b] + t, : pages.numel()] = pages.to(torch.int32)
     ids[:, :, -1] = 10_000  # out of range: ignored
     t32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)  # noqa: E731
+    assert tile_rows(q, k, cq, max(lens_k)) == height
     out = sparse_attention(q.to(DEV), k.to(DEV), v.to(DEV), t32(cq), t32(ck), max(lens_q),
                            max(lens_k), ids.to(DEV))
     rows = sorted(set(spread_rows(cq, per_seq=40)))

@@ -7,7 +7,7 @@ import pytest
 import torch
 
 import oracle
-from gpu_helpers import oracle_select_rows, plan_structure_errors, spread_rows
+from gpu_helpers import oracle_select_rows, plan_structure_errors, spread_rows, tile_rows
 from leanselect_amd import _hip, workloads
 from leanselect_amd.ops import compress_k, leanselect_prefill_topk_idx, sparse_attention
 from leanselect_amd.ops.attention import attention_tile_rows, infllmv2_attn_varlen_func
@@ -253,8 +253,8 @@ def test_attention_tile_sizes_and_tile_deal(lens, biased):
     if biased:
         gen = torch.Generator(device=DEV).manual_seed(15)
         cis = torch.randn(case.cu_host[-1], 2, generator=gen, device=DEV).to(case.q.dtype)
-        out = nosa_sparse_attention(case.q, case.k, case.v, cis, case.cu_seqlens, case.cu_seqlens,
-                                    case.max_seqlen, case.max_seqlen, ids)
+        nosa_sparse_attention(case.q, case.k, case.v, cis, case.cu_seqlens, case.cu_seqlens,
+                              case.max_seqlen, case.max_seqlen, ids, out=out)
         want = oracle.nosa_attention(case.q.cpu(), case.k.cpu(), case.v.cpu(), cis.cpu(),
                                      case.cu_host, case.cu_host, ids.cpu()[:, rows], rows=rows,
                                      ids_rows_aligned=True)
@@ -355,11 +355,17 @@ def test_attention_grid_holds_many_rows_times_groups():
     assert bool((out[rows] == 0).all()) and bool((out[-1] == 0).all())
 
 
-def test_attention_messy_ids_duplicates_unsorted_out_of_range():
-    case, ids = _attention_case(lens=(1500,), seed=7)
+# One sequence per tile height of the launcher (two KV groups).
+EACH_HEIGHT = pytest.mark.parametrize("n,height", [(1500, 8), (3000, 12), (4200, 24)])
+
+
+@EACH_HEIGHT
+def test_attention_messy_ids_duplicates_unsorted_out_of_range(n, height):
+    case, ids = _attention_case(lens=(n,), seed=7)
+    assert tile_rows(case.q, case.k, case.cu_host, n) == height
     g = torch.Generator(device="cpu").manual_seed(0)
     G, N, T = ids.shape
-    messy = torch.randint(-3, 30, (G, N, T), generator=g, dtype=torch.int32)
+    messy = torch.randint(-3, n // 64 + 7, (G, N, T), generator=g, dtype=torch.int32)
     messy[..., 0] = messy[..., 1]  # duplicates
     rows = spread_rows(case.cu_host, per_seq=40)
     _check_attention(case, messy.to(DEV), rows)
@@ -372,8 +378,8 @@ def test_attention_tile_unions_at_their_bound(take, dtype, N):
     """Row r of a 24-row tile takes pages r*take .. r*take + take - 1 (mod the visible
     pages), so at the end of an N-token sequence no two rows of a tile share a page
     and the last full tile's union holds 24 x take pages: 2040, 2304 and 3072 (the
-    bound of the 128-id plans the kernel accepts, past the 2048 pages of a 32-bit
-    need word per lane); earlier rows repeat ids, which the kernel drops."""
+    bound of the 128-id plans the kernel accepts); earlier rows repeat ids, which the
+    kernel drops."""
     case = workloads.hidden_space_layer((N,), device=DEV, dtype=dtype, seed=31)
     G = case.k.shape[1]
     tile = attention_tile_rows(take)
@@ -405,10 +411,13 @@ def test_attention_plans_without_pages(take):
     assert bool(torch.isposinf(lse).all())
 
 
-def test_attention_union_sizes_with_small_factors():
-    """Tiles whose union has 1, 2, 7, 14, 21, 35 or 49 pages (the visit order is a
-    stride permutation of the union, which must stay a bijection for every size)."""
-    case, ids = _attention_case(lens=(4096,), seed=10)
+@pytest.mark.parametrize("n,height", [(1500, 8), (3000, 12), (4096, 24)])
+def test_attention_union_sizes_with_small_factors(n, height):
+    """Groups of 24 rows (whose plans fix the visit order at every tile height) whose
+    union has 1, 2, 7, 14, 21, 35 or 49 pages (the order is a stride permutation of
+    the union, which must stay a bijection for every size)."""
+    case, ids = _attention_case(lens=(n,), seed=10)
+    assert tile_rows(case.q, case.k, case.cu_host, n) == height
     G, N, T = ids.shape
     tile = attention_tile_rows(T)
     crafted = torch.full((G, N, T), -1, dtype=torch.int32)
@@ -421,8 +430,10 @@ def test_attention_union_sizes_with_small_factors():
     _check_attention(case, crafted.to(DEV), rows)
 
 
-def test_attention_group_size_4_and_non_causal():
-    case = workloads.head_space_layer(1024, device=DEV, dtype=torch.bfloat16)
+@pytest.mark.parametrize("n,height", [(1024, 8), (2800, 12), (4200, 24)])
+def test_attention_group_size_4_and_non_causal(n, height):
+    case = workloads.head_space_layer(n, device=DEV, dtype=torch.bfloat16)
+    assert tile_rows(case.q, case.k, case.cu_host, n) == height
     _, _, ids = _select(case)
     rows = spread_rows(case.cu_host, per_seq=40)
     _check_attention(case, ids, rows)
@@ -454,13 +465,15 @@ def test_end_to_end_prefill_32k_sampled():
     assert ok, (mx, mr)
 
 
-def test_ring_wait_expiry_is_reported():
+@EACH_HEIGHT
+def test_ring_wait_expiry_is_reported(n, height):
     """With the wait bound forced to zero from the host every ring wait expires at
     once: the kernel still finishes, the status word is set and the wrapper raises
     (at once with ``sync_status``; at ``attn_status_sync`` otherwise, without the
     call itself waiting), and the rows of the waves whose wait expired are NaN.
     The next call with the default bound is clean and correct."""
-    case, ids = _attention_case(lens=(3000,), seed=4)
+    case, ids = _attention_case(lens=(n,), seed=4)
+    assert tile_rows(case.q, case.k, case.cu_host, n) == height
     L = _hip.lib()
     out = torch.zeros_like(case.q)
     _hip.attn_status_sync()  # nothing earlier is pending
@@ -468,10 +481,10 @@ def test_ring_wait_expiry_is_reported():
     try:
         with pytest.raises(RuntimeError, match="expired"):
             sparse_attention(case.q, case.k, case.v, case.cu_seqlens, case.cu_seqlens,
-                             3000, 3000, ids, out=out, sync_status=True)
+                             n, n, ids, out=out, sync_status=True)
         out2 = torch.zeros_like(case.q)
         sparse_attention(case.q, case.k, case.v, case.cu_seqlens, case.cu_seqlens,
-                         3000, 3000, ids, out=out2)  # deferred: returns without raising
+                         n, n, ids, out=out2)  # deferred: returns without raising
         with pytest.raises(RuntimeError, match="expired"):
             _hip.attn_status_sync()
     finally:
