@@ -16,7 +16,7 @@
 //     with the 8 contiguous keys base+8q..base+8q+7; P^T then feeds the second
 //     MFMA (O^T = V^T . P^T) straight from registers as its B operand and V^T
 //     is read as 16-byte rows of a transposed, page-aligned copy of V built by
-//     ls_vt_kernel (zero-filled past each sequence end);
+//     ls_kv_stage_kernel (zero-filled past each sequence end);
 //   * float32 softmax in base 2; P . V runs on the fp16 MFMA (P in [0, 1]
 //     keeps 10 mantissa bits instead of bf16's 7; V is staged to fp16 with an
 //     exact per-page power-of-two scale that moves onto P), output rounded once.
@@ -80,7 +80,8 @@ __global__ void ls_attn_status_clear_kernel(int32_t* __restrict__ status) {
 // A wave keeps its rows' O^T accumulators (TPW x 8 x 4 floats per lane) and
 // Q^T fragments in registers.  Larger tiles share each page copy among more
 // rows; three rows of O and Q are what the register file holds at two waves per
-// SIMD (with each row reading the chunk's V^T fragments where it uses them).
+// SIMD (254 to 256 registers; the chunk's K and V^T fragments are read once for all
+// rows).
 // ---------------------------------------------------------------------------
 #ifndef LS_ATT_WAVES
 #define LS_ATT_WAVES 8                       // waves per workgroup
@@ -236,10 +237,10 @@ __device__ __forceinline__ float ls_sum_f16x2(uint32_t x, float acc) {
 // kernel took 245.  So the loop keeps a wave's waits off that chain: V^T is read
 // from LDS before the first row's Q K (and once for all rows), the second chunk's
 // K behind the first's softmax, the visit list and the ready word ahead of their
-// use, and the rare branches (causal frontier, rescale) out of line.  Attention
-// alone, same box, before -> after: 13.72 -> 12.19 ms (one 128K sequence, 64
-// pages), 4.00 -> 3.39 ms (32K, 96 pages, few shared), 1.55 -> 1.29 ms (four
-// sequences of 0.5K to 12K), 286 -> 234 us (4K), 3.99 -> 3.58 ms (32K with BIAS).
+// use, and the rare branches (causal frontier, rescale) out of line.  This kernel
+// alone, one box, before -> now: 13.67 -> 12.16 ms (one 128K sequence, 64 pages),
+// 3.99 -> 3.33 ms (32K, 96 pages, few shared), 3.28 -> 2.77 ms (32K with BIAS), 275
+// -> 186 us (4096 rows), 82 -> 38 us (1337 rows, 8-row tiles).
 // BIAS adds a per-key score bias (the NOSA eviction score, pre-scaled to base
 // 2): weight_j = 2^(scale_log2 * q.k_j + cb_j).  cb[g][64 pg_off[b] + j] is
 // staged like V^T and copied with each page (256 B per stage).
@@ -275,8 +276,9 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
   __shared__ int s_wsum[LS_ATT_WAVES];
   // Ring protocol: s_next = next union page to be claimed for copying;
   // s_rdy[st][0] = union index + 1 of the page whose copy into stage st has
-  // landed, s_rdy[st][1] = that page's V exponent (read together); s_done[st] = (union index << 8) | number of its waves done with
-  // it, for the page in stage st (tagged, so a stale count never matches).
+  // landed, s_rdy[st][1] = that page's V exponent (read together); s_done[st] =
+  // (union index << 8) | number of its waves done with it, for the page in stage
+  // st (tagged, so a stale count never matches).
   __shared__ uint32_t s_next, s_done[LS_ATT_STAGES];
   __shared__ __align__(8) uint32_t s_rdy[LS_ATT_STAGES][2];
   __shared__ __align__(16) float s_bias[BIAS ? LS_ATT_STAGES * 64 : 4];
@@ -659,9 +661,9 @@ __global__ __launch_bounds__(LS_ATT_THREADS, LS_ATT_THREADS / 256) void ls_attn_
     }
   };
 
-  // A visit's list entry is read two visits ahead and its stage word during
-  // the visit before, so that neither read is waited for where the page is ready: a page
-  // stays in its stage until this wave is done with it, so a word that showed
+  // A visit's list entry is read two visits ahead and its stage word during the
+  // visit before, so that neither read is waited for where the page is ready: a
+  // page stays in its stage until this wave is done with it, so a word that showed
   // its token once stays valid, and LDS accesses of a wave are in order, so the
   // page's data is read after it.
   auto entry = [&](int k) -> uint32_t { return k < n_visits ? s_wlist[w][k] : 0u; };

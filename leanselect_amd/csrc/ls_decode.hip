@@ -37,14 +37,14 @@ __host__ __device__ __forceinline__ int64_t ls_n_windows(int64_t len, int ks, in
 // thread (row, g, chunk of 8 channels) copies 16 bytes of K and of V to position
 // cache_seqlens[b] + (row - cu_new[b]).  The others form the compressed windows
 // the new tokens complete, the first max_windows of them in the order of the
-// sequences: a pair of threads per (window, g, 8 channels), each summing one half of the window's rows
-// [w*stride, w*stride + ks) in float32 in token order (windows of two strides;
-// other geometries are summed by the first thread alone).  The halves are
-// added, the order of the prefill's half-window kernel, so a window formed here
-// is bit-identical to the one the prefill forms from the same keys.  Rows of
-// this call are read from the new keys rather than the cache, so the windows
-// need not wait for the copies, and each workgroup sums up the batch's new windows
-// itself (256 sequences at a time, in LDS), so they are dealt evenly over
+// sequences: a pair of threads per (window, g, 8 channels), each summing one half
+// of the window's rows [w*stride, w*stride + ks) in float32 in token order
+// (windows of two strides; other geometries are summed by the first thread alone).
+// The halves are added, the order of the prefill's half-window kernel, so a window
+// formed here is bit-identical to the one the prefill forms from the same keys.
+// Rows of this call are read from the new keys rather than the cache, so the
+// windows need not wait for the copies, and each workgroup sums up the batch's new
+// windows itself (256 sequences at a time, in LDS), so they are dealt evenly over
 // the workgroups wherever in the batch they are: what were three launches in a
 // chain are one.  The call, three launches -> one, us: one sequence and one token
 // 18.6 -> 7.0, sixteen 24.1 -> 8.1, 64 sequences of which one gets 64K tokens
@@ -651,8 +651,11 @@ __device__ __forceinline__ void ls_dec_wave_sync() {
 //
 // A wave's pages are pipelined: the next page's K rows are loaded as soon as this
 // page's Q K has read them, its V rows as soon as this page's are in LDS, so a
-// wave's second page does not wait for memory again (no register is added: the
-// loads reuse the fragments they follow).
+// wave's second page does not wait for memory again.  The loads reuse the fragments
+// they follow: 252 to 256 VGPRs and 44 to 49 AGPRs (254 and 32 without the pipeline),
+// at one wave per SIMD either way.  The page's code is there twice, with and without
+// a next page: a first pass on cold caches is no slower for it (16 rows 37.5 us
+// against 38.1 without the pipeline, after 2 GB of other writes).
 // Bound by memory latency at one or two pages a wave, then by the waves' serial
 // page time.  Attention and combine, before -> after: 26.0 -> 21.6 us at four
 // pages a wave (one row of 64 pages, 4 splits), 22.0 -> 21.2 us at two (16 rows).

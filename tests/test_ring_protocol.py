@@ -1,7 +1,7 @@
 """Interleaving model of the attention kernel's LDS copy ring (CPU only).
 
-The tile kernel (leanselect_amd/csrc/ls_attention.hip, ring protocol around
-lines 401-610) streams the tile's union pages through 4 LDS stages.  Union
+The tile kernel (leanselect_amd/csrc/ls_attention.hip, from its "staging" section
+on) streams the tile's union pages through 4 LDS stages.  Union
 page u uses stage u % 4.  Shared state: ``s_next`` (next page to claim),
 ``s_done[st] = (page << 8) | waves done with it`` and the ready token
 ``s_rdy[st] = page + 1``, which a page's copy writes with its final load.
